@@ -224,11 +224,20 @@ def _inputs(case, seed):
     return x, X
 
 
+_work_stream = None
+
+
 class _Plans:
-    """A framework with its plans; both go when the state goes."""
+    """A framework with its plans; both go when the state goes.  Every
+    framework enqueues on the program's one work stream, so transforms of
+    different states run one after the other."""
 
     def __init__(self):
+        global _work_stream
+        if _work_stream is None:
+            _work_stream = torch.cuda.Stream()
         self.fw = topefft.Framework()
+        self.fw.set_stream(_work_stream.cuda_stream)
         self.plans = []
 
     def add(self, plan):
