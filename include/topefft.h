@@ -176,7 +176,9 @@ void topePlanDownload(struct topeFFT *f, void *plan_impl, void *host, size_t byt
 /* Wait for all work enqueued on f->stream. */
 void topeFFTSynchronize(struct topeFFT *f);
 
-/* Number of kernel launches one Exec performs, and per-launch timing:
+/* Number of kernel launches one Exec performs (a length with a prime factor
+ * above 7 and at most 2048 counts chirp_pre and chirp_post, which share one
+ * launch at the position of chirp_pre), and per-launch timing:
  * while enabled, every Exec records HIP events around each launch on
  * f->stream; topePlanPassTimes synchronises and returns the mean duration
  * in milliseconds of each launch position over the recorded execs. */

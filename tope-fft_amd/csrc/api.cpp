@@ -57,6 +57,8 @@ enum PassKind {
     PASS_REAL = 4,
     PASS_CHIRP = 5,
     PASS_MIXED = 6,
+    PASS_CHIRP_LINE = 8,  // Bluestein lines inside a workgroup
+    PASS_DONE = 9,        // a step that the launch before it has carried out
     PASS_RPACK = 7  // real plans: unpack (FORWARD) / pack (INVERSE) of the DC/Nyquist columns
 };
 
@@ -82,6 +84,7 @@ struct Pass {
     long long chirp_n = 0, chirp_M = 0;
     ChirpGeo chirp_g{1, 0, 1, 0, 1};
     const void *chirp_tab[2] = {nullptr, nullptr};  // transformed filters, forward / inverse
+    ChirpLineArgs cl{};                             // PASS_CHIRP_LINE
     MixedArgs mx{};                                 // PASS_MIXED
     const char *name = "";
 };
@@ -98,6 +101,7 @@ struct PlanImpl {
     size_t buf_bytes = 0;  // device arrays when larger than bytes (Bluestein's padded length)
     void *buf[2] = {nullptr, nullptr};
     void *ct3_tw = nullptr;  // twiddle table of the three-step column tiles
+    bool chirpz = false;      // an axis runs Bluestein's convolution
     bool pair_tiles = false;  // a pass moves complex64 column pairs (16-byte aligned arrays)
     int final_buf = 0;
     std::vector<Pass> passes;
@@ -642,7 +646,8 @@ class Planner {
     }
 
     // Non-power-of-two axis of length n (lines g) by Bluestein's identity
-    // (kernels_chirp.hip): chirp pre-multiply of every line into its own
+    // (kernels_chirp.hip).  M <= CHIRP_MAX_M: one in-place pass, each line's
+    // convolution inside a workgroup (bluestein_lines).  Longer: chirp pre-multiply of every line into its own
     // zero-padded row of M elements in the other buffer, forward FFT_M over
     // the rows, product with the transformed filter of the direction,
     // inverse FFT_M (both inner FFTs keep their direction whatever the outer
@@ -730,6 +735,8 @@ class Planner {
         return TOPE_SUCCESS;
     }
 
+    static bool chirp_fused(long long M) { return M >= CHIRP_MIN_M && M <= CHIRP_MAX_M; }
+
     static long long chirp_len(long long n)
     {
         long long M = 1;
@@ -737,9 +744,61 @@ class Planner {
         return M;
     }
 
+    int bluestein_lines(long long n, long long M, const Geo &g, int cur)
+    {
+        void *tab[2] = {nullptr, nullptr}, *ct = nullptr, *tw = nullptr;
+        hipError_t err = stage_table((int)M, 16, &tw);
+        if (err == hipSuccess) err = hipMalloc(&ct, (size_t)n * 16);
+        if (err != hipSuccess) return map_err(err);
+        P->allocs.push_back(ct);
+        err = gen_chirp_table(ct, n, st);
+        for (int d = 0; d < 2 && err == hipSuccess; ++d) {
+            err = hipMalloc(&tab[d], (size_t)M * 16);
+            if (err == hipSuccess) P->allocs.push_back(tab[d]);
+        }
+        if (err != hipSuccess) return map_err(err);
+        // the transformed filters: b into its table, then a one-row forward
+        // FFT_M in place there (planned, run, then dropped from the pass list)
+        const size_t g0 = P->passes.size();
+        int fc = 1;
+        int rc = axis(M, Geo{1, 0, 1, M, 1}, &fc, -1);
+        if (rc) return rc;
+        if (P->passes.size() != g0 + 1 || fc != 1) return TOPE_ERROR_NO_KERNEL;
+        P->passes[g0].a.in_elems = P->passes[g0].a.out_elems = M;
+        void *own1 = P->buf[1];
+        for (int d = 0; d < 2 && !rc; ++d) {
+            P->buf[1] = tab[d];
+            rc = map_err(launch_chirp(CHIRP_FILTER, nullptr, tab[d], nullptr, ChirpGeo{1, 0, 1, 0, 1}, n, M, 1.0, d, st));
+            if (!rc) rc = launch_pass(P, g0, st, FORWARD);
+        }
+        P->buf[1] = own1;
+        P->passes.resize(g0);
+        if (rc) return rc;
+        Pass ps;
+        ps.kind = PASS_CHIRP_LINE;
+        ps.in_buf = ps.out_buf = cur;
+        ps.chirp_tab[0] = tab[0];
+        ps.chirp_tab[1] = tab[1];
+        ps.cl.g = ChirpGeo{g.O, g.os, g.C, g.cs, g.is};
+        ps.cl.n = (int)n;
+        ps.cl.M = (int)M;
+        ps.cl.chirp = ct;
+        ps.cl.tw = tw;
+        ps.name = "chirp_pre";
+        P->passes.push_back(ps);
+        // the axis still reads as running from chirp_pre to chirp_post
+        Pass done;
+        done.kind = PASS_DONE;
+        done.in_buf = done.out_buf = cur;
+        done.name = "chirp_post";
+        P->passes.push_back(done);
+        return TOPE_SUCCESS;
+    }
+
     int bluestein_axis(long long n, const Geo &g, int *cur)
     {
         const long long M = chirp_len(n), lines = g.O * g.C;
+        if (chirp_fused(M)) return bluestein_lines(n, M, g, *cur);
         const int data = *cur, scratch = *cur ^ 1;
         const size_t tb = (size_t)M * 16;
         void *tab[2] = {nullptr, nullptr};
@@ -960,6 +1019,7 @@ hipEvent_t pool_event(PlanImpl *P)
 int launch_pass(PlanImpl *P, size_t i, hipStream_t s, int dir)
 {
     const Pass &ps = P->passes[i];
+    if (ps.kind == PASS_DONE) return TOPE_SUCCESS;
     const int sign = ((ps.fixed_dir >= 0 ? ps.fixed_dir : dir) == FORWARD) ? -1 : 1;
     const double sc = (dir == INVERSE) ? 1.0 / (double)P->norm : 1.0;
     const char *ib = static_cast<const char *>(P->buf[ps.in_buf]);
@@ -995,6 +1055,13 @@ int launch_pass(PlanImpl *P, size_t i, hipStream_t s, int dir)
             hipError_t err = launch_mixed(P->prec, ib + r * ps.rep_in * eb, ob + r * ps.rep_out * eb, m, sign, s);
             if (err != hipSuccess) return map_err(err);
         }
+    } else if (ps.kind == PASS_CHIRP_LINE) {
+        ChirpLineArgs c = ps.cl;
+        c.inverse = dir == INVERSE ? 1 : 0;
+        c.filter = ps.chirp_tab[c.inverse];
+        c.scale = (1.0 / (double)c.M) * (ps.last ? sc : 1.0);
+        hipError_t err = launch_chirp_lines(ib, ob, c, s);
+        if (err != hipSuccess) return map_err(err);
     } else if (ps.kind == PASS_CHIRP) {
         // 1/M undoes the unnormalised inner inverse FFT; the plan's 1/N of
         // INVERSE rides on its last pass as for the axis passes
@@ -1130,6 +1197,8 @@ int build_plan(struct topeFFT *f, int shape, long long nx, long long ny, long lo
                 delete P;
                 return TOPE_ERROR_INVALID_SIZE;
             }
+            P->chirpz = true;
+            if (Planner::chirp_fused(M)) continue;  // in place, no padded rows
             chirpz = true;
             buf_elems = std::max(buf_elems, (size_t)(total / n * M));
         }
@@ -1198,7 +1267,7 @@ int build_plan(struct topeFFT *f, int shape, long long nx, long long ny, long lo
         P->axis_tw[0].table = tw;
     } else if (shape == SHAPE_BATCH) {
         rc = any_axis(pl, nx, Geo{1, 0, ny, nx, 1}, &cur, 0);
-    } else if (nonpow2 && !(shape == 1 && !chirpz && !mixed_supported(nx) && !mixed4(nx))) {
+    } else if (nonpow2 && !(shape == 1 && !P->chirpz && !mixed_supported(nx) && !mixed4(nx))) {
         rc = any_axis(pl, nx, Geo{1, 0, ny * nz, nx, 1}, &cur, 0);
         if (!rc && shape >= 2) rc = any_axis(pl, ny, Geo{nz, nx * ny, nx, 1, nx}, &cur, 1);
         if (!rc && shape >= 3) rc = any_axis(pl, nz, Geo{1, 0, nx * ny, 1, nx * ny}, &cur, 2);
@@ -1236,7 +1305,11 @@ int build_plan(struct topeFFT *f, int shape, long long nx, long long ny, long lo
         if (!rc && shape >= 3) rc = pl.axis(nz, Geo{1, 0, nx * ny, 1, nx * ny}, &cur, 2);
     }
     if (rc) return fail(rc);
-    if (!P->passes.empty()) P->passes.back().last = true;
+    for (size_t i = P->passes.size(); i-- > 0;)  // the last launch
+        if (P->passes[i].kind != PASS_DONE) {
+            P->passes[i].last = true;
+            break;
+        }
     P->final_buf = cur;
     bool need_scratch = false;
     for (const Pass &ps : P->passes)
@@ -2184,8 +2257,8 @@ void topePlanExecPtr(struct topeFFT *f, void *plan_impl, void *data, int dir)
         f->error = TOPE_ERROR_NOT_INITIALIZED;
         return;
     }
-    if (!data || P->real || P->buf_bytes > P->bytes) {
-        // real plans and padded (Bluestein) plans work on arrays of their own
+    if (!data || P->real || P->chirpz) {
+        // real plans and Bluestein plans work on arrays of their own
         f->error = !data ? TOPE_ERROR_INVALID_ARG : TOPE_ERROR_UNSUPPORTED;
         return;
     }

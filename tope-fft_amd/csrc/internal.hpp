@@ -122,6 +122,19 @@ hipError_t launch_mixed(int prec, const void *in, void *out, const MixedArgs &a,
 struct ChirpGeo {
     long long O, os, C, cs, is;
 };
+// The same axis in one pass, each line's convolution inside a workgroup:
+// M = 32 .. CHIRP_MAX_M; chirp holds c[k] (k < n, gen_chirp_table), filter the
+// transformed filter of the direction, tw the stage table of (M, 16).
+constexpr long long CHIRP_MIN_M = 32, CHIRP_MAX_M = 4096;
+struct ChirpLineArgs {
+    ChirpGeo g;
+    long long tiles;  // set by the launcher
+    int n, M, inverse;
+    const void *chirp, *filter, *tw;
+    double scale;  // 1/M, times the plan's 1/N on the last inverse pass
+};
+hipError_t gen_chirp_table(void *out, long long n, hipStream_t st);
+hipError_t launch_chirp_lines(const void *in, void *out, const ChirpLineArgs &a, hipStream_t st);
 hipError_t launch_chirp(int op, const void *in, void *out, const void *table, const ChirpGeo &g, long long n,
                         long long M, double s, int inverse, hipStream_t st);
 // Mixed-precision column tiles (mfma_tile.hpp): 16 unit-stride lines per block.

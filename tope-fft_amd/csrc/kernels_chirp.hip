@@ -11,7 +11,8 @@
 // A = FFT_M(a zero-padded), C = IFFT_M(A * FFT_M(b wrapped)), X[j] = c[j] C[j].
 // The inverse transform uses conj(c) throughout.  Every line of an axis is
 // padded into its own row of M elements of a scratch array, so the two inner
-// FFTs are contiguous row passes.
+// FFTs are contiguous row passes.  Up to M = CHIRP_MAX_M a line's whole
+// convolution runs in one workgroup instead (chirp_line_kernel).
 #include "internal.hpp"
 
 namespace tope {
@@ -41,6 +42,86 @@ __global__ void chirp_filter_kernel(cpx<double> *b, long long n, long long M, in
         v = cpx<double>{c.x, -c.y};
     }
     b[i] = v;
+}
+
+// c[k] = W_2n^(k^2), k < n, forward sign.
+__global__ void chirp_table_kernel(cpx<double> *c, long long n)
+{
+    const long long k = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (k < n) c[k] = chirp(k, n, 0);
+}
+
+// One axis of lines of length n, M = N >= 2n - 1, in one launch: a block
+// takes TB lines, multiplies them by the chirp as it loads them, runs the
+// forward FFT_M, the product with the transformed filter and the inverse
+// FFT_M in registers with LDS exchanges (run_stages), and stores the n
+// outputs times the chirp.  In place, no padded array: an element is read
+// and written once, where the separate passes moved 2 + 8 M/n elements per
+// element through memory and evaluated a sincospi at both ends.  2D
+// 1009 x 1009 (M = 2048): 133 us in ten launches -> 36 us in two.
+//
+// Each thread holds elements p + P e (P = N/16): n <= M/2, so those with
+// e >= 8 are padding on the way in and unused on the way out.  Rows put the
+// P threads of a line on neighbouring lanes; strided axes put TB adjacent
+// lines there.  The real and imaginary parts are exchanged in turn, which
+// halves the LDS of a tile, except in rows of M >= 2048, which fit four
+// blocks per CU whole (1999 x 251: 52.1 -> 51.3 us, both for a forward and an
+// inverse transform).  What bounds it now is the latency of its two serial
+// transforms at two to three waves per SIMD (160-190 VGPRs): four waves
+// (128 VGPRs) measured slower, 63 -> 82 us at 251 x 1999 and 52 -> 71 us at
+// 1999 x 251, and leaving out the additions of the zero half changed nothing.
+template <int N, int TB, bool CFAST>
+__global__ void __launch_bounds__(TB *(N / 16))
+chirp_line_kernel(const cpx<double> *in, cpx<double> *out, const ChirpLineArgs a)
+{
+    using R = double;
+    constexpr int E = 16, P = N / E, H = E / 2;
+    constexpr bool SPLIT = CFAST || N < 2048;
+    __shared__ __align__(16) unsigned char lds[Exchange<R, N, E, TB, CFAST, SPLIT>::BYTES];
+    const int tid = threadIdx.x;
+    const int t = CFAST ? tid % TB : tid / P;
+    const int p = CFAST ? tid / TB : tid % P;
+    const cpx<R> *tw = static_cast<const cpx<R> *>(a.tw);
+    const cpx<R> *ct = static_cast<const cpx<R> *>(a.chirp);
+    const cpx<R> *fl = static_cast<const cpx<R> *>(a.filter);
+
+    const long long blk = xcd_block(CFAST ? 1 : 0);
+    const long long o = blk / a.tiles;
+    const long long c = (blk - o * a.tiles) * TB + t;
+    const bool valid = c < a.g.C;
+    const long long at = o * a.g.os + c * a.g.cs;
+
+    cpx<R> v[E];
+#pragma unroll
+    for (int e = 0; e < H; ++e) {
+        const int k = p + P * e;
+        v[e] = valid && k < a.n ? in[at + k * a.g.is] : cpx<R>{0, 0};
+    }
+#pragma unroll
+    for (int e = 0; e < H; ++e) {
+        const int k = p + P * e;
+        const cpx<R> w = ct[k < a.n ? k : 0];
+        v[e] = a.inverse ? cmulc(v[e], w) : cmul(v[e], w);
+    }
+#pragma unroll
+    for (int e = H; e < E; ++e) v[e] = cpx<R>{0, 0};
+
+    run_stages<R, N, E, TB, CFAST, SPLIT, -1, 0>(v, p, t, tw, lds);
+#pragma unroll
+    for (int e = 0; e < E; ++e) v[e] = cmul(v[e], fl[p + P * e]);
+    __syncthreads();  // the forward transform's last exchange has been read
+    run_stages<R, N, E, TB, CFAST, SPLIT, 1, 0>(v, p, t, tw, lds);
+
+    if (!valid) return;
+#pragma unroll
+    for (int e = 0; e < H; ++e) {
+        const int k = p + P * e;
+        if (k < a.n) {
+            const cpx<R> w = ct[k];
+            const cpx<R> r = a.inverse ? cmulc(v[e], w) : cmul(v[e], w);
+            out[at + k * a.g.is] = cpx<R>{r.x * a.scale, r.y * a.scale};
+        }
+    }
 }
 
 // Element k of line l (o = l / C, c = l % C) of the axis: o os + c cs + k is.
@@ -94,6 +175,51 @@ __global__ void chirp_post_kernel(const cpx<double> *__restrict__ S, cpx<double>
     line_of(idx, g, n, l, j);
     const cpx<double> v = cmul(S[l * M + j], chirp(j, n, inverse));
     x[elem_of(l, j, g)] = cpx<double>{v.x * s, v.y * s};
+}
+
+template <int N, int TB, bool CFAST>
+static hipError_t launch_line_t(const void *in, void *out, ChirpLineArgs a, hipStream_t st)
+{
+    a.tiles = (a.g.C + TB - 1) / TB;
+    const long long grid = a.g.O * a.tiles;
+    if (grid < 1 || grid > 0x7fffffffLL) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((chirp_line_kernel<N, TB, CFAST>), dim3((unsigned)grid), dim3(TB * (N / 16)), 0, st,
+                       static_cast<const cpx<double> *>(in), static_cast<cpx<double> *>(out), a);
+    return hipGetLastError();
+}
+
+// Rows: 64 to 256 threads a block.  Strided axes: tiles of WIDE adjacent
+// lines (64-byte segments or more), or NARROW ones where the wide tiles
+// would leave CUs with no more than one block.
+template <int N, int ROW, int WIDE, int NARROW>
+static hipError_t launch_line_n(const void *in, void *out, const ChirpLineArgs &a, hipStream_t st)
+{
+    if (a.g.is == 1) return launch_line_t<N, ROW, false>(in, out, a, st);
+    if (a.g.O * ((a.g.C + WIDE - 1) / WIDE) < 512) return launch_line_t<N, NARROW, true>(in, out, a, st);
+    return launch_line_t<N, WIDE, true>(in, out, a, st);
+}
+
+hipError_t launch_chirp_lines(const void *in, void *out, const ChirpLineArgs &a, hipStream_t st)
+{
+    if (a.n < 1 || 2LL * a.n - 1 > a.M) return hipErrorInvalidValue;
+    switch (a.M) {
+    case 32: return launch_line_n<32, 32, 32, 32>(in, out, a, st);
+    case 64: return launch_line_n<64, 16, 16, 16>(in, out, a, st);
+    case 128: return launch_line_n<128, 16, 16, 8>(in, out, a, st);
+    case 256: return launch_line_n<256, 8, 16, 4>(in, out, a, st);
+    case 512: return launch_line_n<512, 4, 8, 4>(in, out, a, st);
+    case 1024: return launch_line_n<1024, 2, 8, 4>(in, out, a, st);
+    case 2048: return launch_line_n<2048, 1, 4, 2>(in, out, a, st);
+    case 4096: return launch_line_n<4096, 1, 4, 2>(in, out, a, st);
+    default: return hipErrorInvalidValue;
+    }
+}
+
+hipError_t gen_chirp_table(void *out, long long n, hipStream_t st)
+{
+    hipLaunchKernelGGL(chirp_table_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st,
+                       static_cast<cpx<double> *>(out), n);
+    return hipGetLastError();
 }
 
 static unsigned grid_of(long long count) { return (unsigned)((count + 255) / 256); }
