@@ -668,20 +668,17 @@ class Planner {
         long long S = 1;
         while (S * S < n) ++S;
         void *r1 = nullptr, *r2 = nullptr, *lo = nullptr, *hi = nullptr;
-        hipError_t err = power_table(N2, 1, N2, &r1);
-        if (err == hipSuccess) err = power_table(N1, 1, N1, &r2);
-        if (err == hipSuccess) err = power_table(n, 1, S, &lo);
+        hipError_t err = power_table(n, 1, S, &lo);
         if (err == hipSuccess) err = power_table(n, S, (n + S - 1) / S, &hi);
         if (err != hipSuccess) return map_err(err);
         auto mixed_pass = [&](long long len, const Fold &f, long long in_is, long long out_is, int bi, int bo,
-                              const void *roots, bool post) {
+                              void **roots, bool post) -> int {
             Pass ps;
             ps.kind = PASS_MIXED;
             ps.mx = mixed_plan(len, f.in.O, f.in.os, f.in.C, f.in.cs, in_is);
             ps.mx.oos = f.out.os;
             ps.mx.ocs = f.out.cs;
             ps.mx.ois = out_is;
-            ps.mx.roots = roots;
             if (post) {
                 ps.mx.pt_lo = lo;
                 ps.mx.pt_hi = hi;
@@ -690,6 +687,8 @@ class Planner {
                 ps.mx.pt_c = f.new_in_c ? 1 : 0;
                 ps.mx.pt_split = (int)S;
             }
+            int rc = mixed_tables(ps.mx, roots);
+            if (rc) return rc;
             ps.grid = mixed_grid(ps.mx);
             ps.in_buf = bi;
             ps.out_buf = bo;
@@ -698,11 +697,13 @@ class Planner {
             ps.rep_out = f.rep_out;
             ps.name = P->prec == PREC_F64 ? "mixed_radix_f64" : "mixed_radix_f32";
             P->passes.push_back(ps);
+            return TOPE_SUCCESS;
         };
         // step 1: lines (old o, old c, n1)
-        mixed_pass(N2, fold(g, N1, g.is, g.is), N1 * g.is, N1 * g.is, *cur, *cur ^ 1, r1, true);
+        int rc = mixed_pass(N2, fold(g, N1, g.is, g.is), N1 * g.is, N1 * g.is, *cur, *cur ^ 1, &r1, true);
         // step 2: lines (old o, old c, k2)
-        mixed_pass(N1, fold(g, N2, N1 * g.is, g.is), g.is, N2 * g.is, *cur ^ 1, *cur, r2, false);
+        if (!rc) rc = mixed_pass(N1, fold(g, N2, N1 * g.is, g.is), g.is, N2 * g.is, *cur ^ 1, *cur, &r2, false);
+        if (rc) return rc;
         if (axis_id >= 0 && !P->axis_tw[axis_id].table) {
             P->axis_tw[axis_id].n = (int)N2;
             P->axis_tw[axis_id].e = 0;
@@ -711,18 +712,34 @@ class Planner {
         return TOPE_SUCCESS;
     }
 
+    // Radices, tile and tables of a mixed-radix pass whose geometry is set:
+    // W_n^i (i < n, *roots), then the stage table, in one allocation.
+    int mixed_tables(MixedArgs &m, void **roots)
+    {
+        mixed_schedule(m, P->prec);
+        void *d = nullptr;
+        hipError_t err = hipMalloc(&d, (size_t)(m.n + m.twsize) * P->elem);
+        if (err != hipSuccess) return map_err(err);
+        P->allocs.push_back(d);
+        err = gen_power_table(d, P->prec, m.n, 1, m.n, st);
+        void *tw = static_cast<char *>(d) + (size_t)m.n * P->elem;
+        if (err == hipSuccess) err = gen_mixed_table(tw, d, P->prec, m, st);
+        m.tw = tw;
+        *roots = d;
+        return map_err(err);
+    }
+
     // Axis of 7-smooth length n <= 4096 that is not a power of two: one
-    // in-place mixed-radix pass (kernels_mixed.hip), twiddles and radix-3/5/7
-    // constants from a table of W_n^i.
+    // in-place mixed-radix pass (kernels_mixed.hip), twiddles from a table of
+    // W_n^i.
     int mixed_axis(long long n, const Geo &g, int cur, int axis_id)
     {
         void *roots = nullptr;
-        hipError_t err = power_table(n, 1, n, &roots);
-        if (err != hipSuccess) return map_err(err);
         Pass ps;
         ps.kind = PASS_MIXED;
         ps.mx = mixed_plan(n, g.O, g.os, g.C, g.cs, g.is);
-        ps.mx.roots = roots;
+        int rc = mixed_tables(ps.mx, &roots);
+        if (rc) return rc;
         ps.grid = mixed_grid(ps.mx);
         ps.in_buf = ps.out_buf = cur;
         ps.name = P->prec == PREC_F64 ? "mixed_radix_f64" : "mixed_radix_f32";
@@ -748,14 +765,12 @@ class Planner {
     {
         void *tab[2] = {nullptr, nullptr}, *ct = nullptr, *tw = nullptr;
         hipError_t err = stage_table((int)M, 16, &tw);
-        if (err == hipSuccess) err = hipMalloc(&ct, (size_t)n * 16);
+        if (err == hipSuccess) err = hipMalloc(&tab[0], (size_t)(2 * M + n) * 16);
         if (err != hipSuccess) return map_err(err);
-        P->allocs.push_back(ct);
+        P->allocs.push_back(tab[0]);
+        tab[1] = static_cast<char *>(tab[0]) + M * 16;
+        ct = static_cast<char *>(tab[1]) + M * 16;
         err = gen_chirp_table(ct, n, st);
-        for (int d = 0; d < 2 && err == hipSuccess; ++d) {
-            err = hipMalloc(&tab[d], (size_t)M * 16);
-            if (err == hipSuccess) P->allocs.push_back(tab[d]);
-        }
         if (err != hipSuccess) return map_err(err);
         // the transformed filters: b into its table, then a one-row forward
         // FFT_M in place there (planned, run, then dropped from the pass list)

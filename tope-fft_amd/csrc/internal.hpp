@@ -92,16 +92,26 @@ hipError_t launch_real_pack(int prec, int dir, void *X, long long m, long long p
 // (o < O, c < C) of the axis sit at o os + c cs, elements is apart, and
 // line l is padded into row l of an M-element-row scratch array.
 enum { CHIRP_FILTER = 0, CHIRP_PRE = 1, CHIRP_MUL = 2, CHIRP_POST = 3 };
-// Mixed-radix (2, 3, 4, 5, 7, 8, 16) in-place axis pass for 7-smooth
-// lengths up to MIXED_MAX_N (kernels_mixed.hip), FP64: line l = o C + c
-// (o < O, c < C) starts at o os + c cs, its elements are `is` apart; roots
-// holds W_n^i, i < n (forward sign).
+// Mixed-radix (2 .. 16) in-place axis pass for 7-smooth lengths up to
+// MIXED_MAX_N (kernels_mixed.hip): line l = o C + c (o < O, c < C) starts at
+// o os + c cs, its elements are `is` apart.
 constexpr int MIXED_MAX_N = 4096;
+constexpr int MIXED_MAX_STAGES = 8;
+struct MixedStage {
+    int r, nb, Ns;  // radix, butterflies per line, span
+    int tw;         // first entry of the stage in the table
+    float inv_nb, inv_Ns;
+};
 struct MixedArgs {
     long long O, os, C, cs, is, lines;
-    int n, tb, nst;
-    int radix[16];
-    const void *roots;  // W_n^i, i < n, in the pass's precision (forward sign)
+    int n, nst;
+    MixedStage st[MIXED_MAX_STAGES];
+    int cap;         // elements a thread can hold at the list's radices
+    int twsize;      // entries of the stage table
+    int nt, tb;      // threads and lines per block
+    float inv_tb;
+    double inv_C;
+    const void *tw;  // stage table (gen_mixed_table), in the pass's precision
     double scale;
     // output geometry (mixed_plan sets it equal to the input's)
     long long oos, ocs, ois;
@@ -111,12 +121,18 @@ struct MixedArgs {
     const void *pt_lo, *pt_hi;
     long long pt_n, pt_o, pt_c;
     int pt_split;
+    float inv_split;
 };
 bool mixed_supported(long long n);
 // 7-smooth n above MIXED_MAX_N that splits as n = n1 n2 with both factors
 // at most MIXED_MAX_N (mixed-radix four-step); *n1 >= n2 is the split used.
 bool mixed4_split(long long n, long long *n1);
+// Arguments with the geometry; mixed_schedule adds the radices and the tile once
+// the output geometry and the post-twiddle are set.
 MixedArgs mixed_plan(long long n, long long O, long long os, long long C, long long cs, long long is);
+void mixed_schedule(MixedArgs &a, int prec);
+// a.twsize stage twiddles from the table W_n^i, i < n (forward sign)
+hipError_t gen_mixed_table(void *out, const void *roots, int prec, const MixedArgs &a, hipStream_t st);
 unsigned mixed_grid(const MixedArgs &a);
 hipError_t launch_mixed(int prec, const void *in, void *out, const MixedArgs &a, int sign, hipStream_t st);
 struct ChirpGeo {

@@ -1,0 +1,46 @@
+// The mixed-radix kernels of one precision and one direction, for real type
+// MIXED_R and sign MIXED_SIGN: compiled once for each of the four.
+#include "mixed_kernel.hpp"
+
+namespace tope {
+
+template <typename R, int SIGN, int NT, bool COL, bool POST>
+static void launch(const void *in, void *out, const MixedArgs &a, unsigned grid, hipStream_t st)
+{
+    const size_t slots = (size_t)mixed_slots<COL>(a.n, a.tb);
+    hipLaunchKernelGGL((mixed_kernel<R, SIGN, NT, COL, POST>), dim3(grid), dim3(NT), slots * sizeof(cpx<R>), st,
+                       static_cast<const cpx<R> *>(in), static_cast<cpx<R> *>(out), a);
+}
+
+template <typename R, int SIGN, int NT>
+static void launch_nt(const void *in, void *out, const MixedArgs &a, unsigned grid, hipStream_t st)
+{
+    const bool col = a.is != 1 || a.ois != 1;  // the planner's post-twiddle passes are strided
+    if (a.pt_n) launch<R, SIGN, NT, true, true>(in, out, a, grid, st);
+    else if (col) launch<R, SIGN, NT, true, false>(in, out, a, grid, st);
+    else if constexpr (NT <= 512) launch<R, SIGN, NT, false, false>(in, out, a, grid, st);
+}
+
+template <typename R, int SIGN>
+hipError_t launch_mixed_t(const void *in, void *out, const MixedArgs &a, unsigned grid, hipStream_t st)
+{
+    if (a.nst == 1) {
+        const cpx<R> *i = static_cast<const cpx<R> *>(in);
+        cpx<R> *o = static_cast<cpx<R> *>(out);
+        if (a.pt_n) hipLaunchKernelGGL((mixed_one_kernel<R, SIGN, true>), dim3(grid), dim3(256), 0, st, i, o, a);
+        else hipLaunchKernelGGL((mixed_one_kernel<R, SIGN, false>), dim3(grid), dim3(256), 0, st, i, o, a);
+        return hipGetLastError();
+    }
+    switch (a.nt) {
+    case 128: launch_nt<R, SIGN, 128>(in, out, a, grid, st); break;
+    case 256: launch_nt<R, SIGN, 256>(in, out, a, grid, st); break;
+    case 512: launch_nt<R, SIGN, 512>(in, out, a, grid, st); break;
+    case 1024: launch_nt<R, SIGN, 1024>(in, out, a, grid, st); break;
+    default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+
+template hipError_t launch_mixed_t<MIXED_R, MIXED_SIGN>(const void *, void *, const MixedArgs &, unsigned, hipStream_t);
+
+}  // namespace tope
