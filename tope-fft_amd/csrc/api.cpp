@@ -72,7 +72,8 @@ struct Pass {
     int mfma_mode = 0, mfma_n = 0;
     unsigned grid = 0;
     int in_buf = 0, out_buf = 0;
-    long long reps = 1, rep_in = 0, rep_out = 0;  // repeated launches (rare geometry)
+    long long reps = 1, rep_in = 0, rep_out = 0;  // repeated launches, their element offsets
+    int group = 0;  // != 0: neighbours of one group run their launches in turn (chunks)
     long long base = 0;                           // element offset of the pass's geometry in both buffers
     bool last = false;                            // receives the inverse 1/N scale
     long long dft_n = 0;
@@ -310,7 +311,7 @@ const AxisVariant *select_variant(int prec, int n, bool cfast, long long lines, 
     return best;
 }
 
-int launch_pass(PlanImpl *P, size_t i, hipStream_t s, int dir);
+int launch_pass(PlanImpl *P, size_t i, hipStream_t s, int dir, long long rep0 = 0, long long rep1 = -1);
 
 struct Geo {  // lines (o < O, c < C) of length n, element stride is
     long long O, os, C, cs, is;
@@ -1030,8 +1031,9 @@ hipEvent_t pool_event(PlanImpl *P)
     return P->pool[P->pool_used++];
 }
 
-// Launch pass i of a plan on stream s.
-int launch_pass(PlanImpl *P, size_t i, hipStream_t s, int dir)
+// Launch pass i of a plan on stream s: its repetitions rep0 .. rep1 - 1, all
+// of them if rep1 < 0.
+int launch_pass(PlanImpl *P, size_t i, hipStream_t s, int dir, long long rep0, long long rep1)
 {
     const Pass &ps = P->passes[i];
     if (ps.kind == PASS_DONE) return TOPE_SUCCESS;
@@ -1040,33 +1042,47 @@ int launch_pass(PlanImpl *P, size_t i, hipStream_t s, int dir)
     const char *ib = static_cast<const char *>(P->buf[ps.in_buf]);
     char *ob = static_cast<char *>(P->buf[ps.out_buf]);
     const long long eb = (long long)P->elem;
+    if (rep1 < 0) rep1 = ps.reps;
     if (ps.kind == PASS_AXIS) {
         if (ps.var->prec == PREC_F64) {
             AxisArgs<double> a = ps.a;
             a.scale = ps.last ? sc : 1.0;
             a.in_elems -= ps.base;
             a.out_elems -= ps.base;
-            for (long long r = 0; r < ps.reps; ++r)
+            const long long ie = a.in_elems, oe = a.out_elems;
+            for (long long r = rep0; r < rep1; ++r) {
+                a.in_elems = ie - r * ps.rep_in;
+                a.out_elems = oe - r * ps.rep_out;
                 ps.var->fn(ib + (ps.base + r * ps.rep_in) * eb, ob + (ps.base + r * ps.rep_out) * eb, &a, ps.grid, s,
                            sign);
+            }
         } else {
             AxisArgs<float> a = ps.a32;
             a.scale = ps.last ? (float)sc : 1.0f;
             a.in_elems -= ps.base;
             a.out_elems -= ps.base;
-            for (long long r = 0; r < ps.reps; ++r)
+            const long long ie = a.in_elems, oe = a.out_elems;
+            for (long long r = rep0; r < rep1; ++r) {
+                a.in_elems = ie - r * ps.rep_in;
+                a.out_elems = oe - r * ps.rep_out;
                 ps.var->fn(ib + (ps.base + r * ps.rep_in) * eb, ob + (ps.base + r * ps.rep_out) * eb, &a, ps.grid, s,
                            sign);
+            }
         }
     } else if (ps.kind == PASS_MFMA) {
         MfmaArgs m = ps.m;
         m.scale = ps.last ? (float)sc : 1.0f;  // 1/N is a power of two: exact in FP32
-        hipError_t err = launch_mfma_rows(ps.mfma_mode, ps.mfma_n, ib, ob, m, sign, s);
-        if (err != hipSuccess) return map_err(err);
+        const long long ie = m.in_elems;
+        for (long long r = rep0; r < rep1; ++r) {
+            m.in_elems = m.out_elems = ie - r * ps.rep_in;
+            hipError_t err =
+                launch_mfma_rows(ps.mfma_mode, ps.mfma_n, ib + r * ps.rep_in * eb, ob + r * ps.rep_out * eb, m, sign, s);
+            if (err != hipSuccess) return map_err(err);
+        }
     } else if (ps.kind == PASS_MIXED) {
         MixedArgs m = ps.mx;
         m.scale = ps.last ? sc : 1.0;
-        for (long long r = 0; r < ps.reps; ++r) {
+        for (long long r = rep0; r < rep1; ++r) {
             hipError_t err = launch_mixed(P->prec, ib + r * ps.rep_in * eb, ob + r * ps.rep_out * eb, m, sign, s);
             if (err != hipSuccess) return map_err(err);
         }
@@ -1087,14 +1103,17 @@ int launch_pass(PlanImpl *P, size_t i, hipStream_t s, int dir)
         if (err != hipSuccess) return map_err(err);
     } else if (ps.kind == PASS_REAL) {
         const bool fwd = dir == FORWARD;
-        const void *src = P->buf[fwd ? ps.in_buf : ps.out_buf];
-        void *dst = P->buf[fwd ? ps.out_buf : ps.in_buf];
-        hipError_t err =
-            ps.real_stw ? launch_real_rows(P->prec, fwd ? 0 : 1, src, dst, ps.real_stw, ps.real_w, P->real_m, P->real_pitch,
-                                           P->real_rows, P->real_scale, P->real_pack ? 1 : 0, s)
-                        : launch_real_pass(P->prec, fwd ? 0 : 1, src, dst, ps.real_w, P->real_m, P->real_pitch, P->real_rows,
-                                           P->real_scale, P->real_pack ? 1 : 0, s);
-        if (err != hipSuccess) return map_err(err);
+        const long long rows = P->real_rows / ps.reps;
+        for (long long r = rep0; r < rep1; ++r) {
+            const char *src = fwd ? ib + r * ps.rep_in * eb : ob + r * ps.rep_out * eb;
+            char *dst = fwd ? ob + r * ps.rep_out * eb : const_cast<char *>(ib) + r * ps.rep_in * eb;
+            hipError_t err =
+                ps.real_stw ? launch_real_rows(P->prec, fwd ? 0 : 1, src, dst, ps.real_stw, ps.real_w, P->real_m,
+                                               P->real_pitch, rows, P->real_scale, P->real_pack ? 1 : 0, s)
+                            : launch_real_pass(P->prec, fwd ? 0 : 1, src, dst, ps.real_w, P->real_m, P->real_pitch, rows,
+                                               P->real_scale, P->real_pack ? 1 : 0, s);
+            if (err != hipSuccess) return map_err(err);
+        }
     } else if (ps.kind == PASS_RPACK) {
         hipError_t err = launch_real_pack(P->prec, dir == FORWARD ? 0 : 1, P->buf[ps.in_buf], P->real_m, P->real_pitch,
                                           P->dims[1], P->dims[2], s);
@@ -1102,8 +1121,13 @@ int launch_pass(PlanImpl *P, size_t i, hipStream_t s, int dir)
     } else if (ps.kind == PASS_MFMA_TILE) {
         MfmaTileArgs m = ps.mt;
         m.scale = ps.last ? (float)sc : 1.0f;
-        hipError_t err = launch_mfma_tile(ps.mfma_mode, ps.mfma_n, ib, ob, m, ps.grid, sign, s);
-        if (err != hipSuccess) return map_err(err);
+        const long long ie = m.in_elems;
+        for (long long r = rep0; r < rep1; ++r) {
+            m.in_elems = m.out_elems = ie - r * ps.rep_in;
+            hipError_t err = launch_mfma_tile(ps.mfma_mode, ps.mfma_n, ib + r * ps.rep_in * eb,
+                                              ob + r * ps.rep_out * eb, m, ps.grid, sign, s);
+            if (err != hipSuccess) return map_err(err);
+        }
     } else {
         hipError_t err = launch_naive_dft(P->prec, ib, ob, ps.dft_roots, ps.dft_n, sign, ps.last ? sc : 1.0, s);
         if (err != hipSuccess) return map_err(err);
@@ -1125,7 +1149,19 @@ int enqueue(PlanImpl *P, hipStream_t s, int dir)
             if (!e0 || !e1) return TOPE_ERROR_UNSUPPORTED;
             (void)hipEventRecord(e0, s);
         }
-        int rc = launch_pass(P, i, s, dir);
+        int rc = TOPE_SUCCESS;
+        if (P->passes[i].group && !P->timing) {
+            // the group's passes chunk by chunk
+            const int g = P->passes[i].group;
+            size_t e = n;
+            while (e < P->passes.size() && P->passes[rev ? (size_t)P->inv_order[e] : e].group == g) ++e;
+            for (long long r = 0; r < P->passes[i].reps && !rc; ++r)
+                for (size_t k = n; k < e && !rc; ++k)
+                    rc = launch_pass(P, rev ? (size_t)P->inv_order[k] : k, s, dir, r, r + 1);
+            n = e - 1;
+        } else {
+            rc = launch_pass(P, i, s, dir);
+        }
         if (rc) return rc;
         if (P->timing) {
             (void)hipEventRecord(e1, s);
@@ -1146,6 +1182,26 @@ void sync_fields(Plan *t, PlanImpl *P)
 PlanImpl *impl_of(void *p) { return static_cast<PlanImpl *>(p); }
 
 enum { SHAPE_BATCH = 4 };
+
+// Planes of a volume that the X and Y passes take at a time.  Beyond the 256
+// MB Infinity Cache the Y pass would read back from memory what the X pass
+// wrote; over chunks that fill the cache it finds part of it there: 512^3
+// complex64 2416 -> 2212 us, 512^3 FP64 4826 -> 4420 us, 512 x 512 x 256
+// complex64 (512 MiB) 1175 -> 1074 us for a forward and an inverse transform.
+// Smaller chunks lose more at the kernel boundaries (about 6 us each) than
+// they find in the cache: 128 MiB 2330 us, 64 MiB 2566 us at 512^3 complex64;
+// 512 MiB 2454 us.  Real plans (the spectrum's planes) gain 3-4 % at 512^3 and
+// lose 7 % at 512 x 256 x 256, whose spectrum is just larger than the cache.
+// All planes at once below twice the cache, or when no divisor of nz gives
+// half of it.
+constexpr long long kCacheBytes = 256LL << 20;
+long long cache_planes(long long nz, long long plane_bytes)
+{
+    if (nz * plane_bytes < 2 * kCacheBytes) return nz;
+    for (long long z = std::min(nz, kCacheBytes / plane_bytes); z >= 1; --z)
+        if (nz % z == 0) return z * plane_bytes >= kCacheBytes / 2 ? z : nz;
+    return nz;
+}
 
 // Common plan construction.  shape 1/2/3: an nx*ny*nz FP64 array (the
 // reference plans); SHAPE_BATCH: ny rows of length nx in precision `prec`
@@ -1254,6 +1310,18 @@ int build_plan(struct topeFFT *f, int shape, long long nx, long long ny, long lo
     Planner pl(P, s);
     pl.flip = true;  // the plan swaps its buffers when the data ends in buffer 1
     int cur = 0, rc = TOPE_SUCCESS;
+    // 3D arrays beyond the cache: X and Y passes in turn over zc planes
+    auto one_pass = [](long long n) { return n <= kMaxFused && (is_pow2(n) || mixed_supported(n)); };
+    const long long zc =
+        shape == 3 && one_pass(nx) && one_pass(ny) ? cache_planes(nz, nx * ny * (long long)P->elem) : nz;
+    auto chunked = [&]() {
+        if (zc == nz) return;
+        for (Pass &ps : P->passes) {
+            ps.group = 1;
+            ps.reps = nz / zc;
+            ps.rep_in = ps.rep_out = zc * nx * ny;
+        }
+    };
     if (shape == SHAPE_BATCH && mode != MP_VALU) {
         // one MFMA launch over all rows, in place
         void *tw = nullptr, *kc = nullptr;
@@ -1283,8 +1351,9 @@ int build_plan(struct topeFFT *f, int shape, long long nx, long long ny, long lo
     } else if (shape == SHAPE_BATCH) {
         rc = any_axis(pl, nx, Geo{1, 0, ny, nx, 1}, &cur, 0);
     } else if (nonpow2 && !(shape == 1 && !P->chirpz && !mixed_supported(nx) && !mixed4(nx))) {
-        rc = any_axis(pl, nx, Geo{1, 0, ny * nz, nx, 1}, &cur, 0);
-        if (!rc && shape >= 2) rc = any_axis(pl, ny, Geo{nz, nx * ny, nx, 1, nx}, &cur, 1);
+        rc = any_axis(pl, nx, Geo{1, 0, ny * zc, nx, 1}, &cur, 0);
+        if (!rc && shape >= 2) rc = any_axis(pl, ny, Geo{zc, nx * ny, nx, 1, nx}, &cur, 1);
+        if (!rc) chunked();
         if (!rc && shape >= 3) rc = any_axis(pl, nz, Geo{1, 0, nx * ny, 1, nx * ny}, &cur, 2);
     } else if (shape == 1 && !is_pow2(nx)) {
         // short non-power-of-two 1D: GPU DFT with exactly reduced phases
@@ -1308,15 +1377,17 @@ int build_plan(struct topeFFT *f, int shape, long long nx, long long ny, long lo
         P->axis_tw[0].table = roots;
     } else if (mode != MP_VALU) {
         // complex64 on the matrix cores where a kernel covers the axis
-        rc = pl.axis_mp(nx, Geo{1, 0, ny * nz, nx, 1}, &cur, 0, mode);
-        if (!rc) rc = pl.axis_mp(ny, Geo{nz, nx * ny, nx, 1, nx}, &cur, 1, mode);
+        rc = pl.axis_mp(nx, Geo{1, 0, ny * zc, nx, 1}, &cur, 0, mode);
+        if (!rc) rc = pl.axis_mp(ny, Geo{zc, nx * ny, nx, 1, nx}, &cur, 1, mode);
+        if (!rc) chunked();
         if (!rc && shape >= 3) rc = pl.axis_mp(nz, Geo{1, 0, nx * ny, 1, nx * ny}, &cur, 2, mode);
     } else if (shape == 2 && nx <= kMaxFused && ny <= kMaxFused && ny >= 4 && ny >= dif2_min_rows()) {
         rc = pl.plan_2d_dif2(nx, ny, &cur);
     } else {
         // X: rows; Y: columns of each plane; Z: columns of the whole volume
-        rc = pl.axis(nx, Geo{1, 0, ny * nz, nx, 1}, &cur, 0);
-        if (!rc && shape >= 2) rc = pl.axis(ny, Geo{nz, nx * ny, nx, 1, nx}, &cur, 1);
+        rc = pl.axis(nx, Geo{1, 0, ny * zc, nx, 1}, &cur, 0);
+        if (!rc && shape >= 2) rc = pl.axis(ny, Geo{zc, nx * ny, nx, 1, nx}, &cur, 1);
+        if (!rc) chunked();
         if (!rc && shape >= 3) rc = pl.axis(nz, Geo{1, 0, nx * ny, 1, nx * ny}, &cur, 2);
     }
     if (rc) return fail(rc);
@@ -1496,7 +1567,19 @@ int build_real_plan(struct topeFFT *f, long long nx, long long ny, long long nz,
             group_end.push_back(P->passes.size());
             return (int)TOPE_SUCCESS;
         };
-        rc = axis2(ny, Geo{nz, pitch * ny, cols, 1, pitch}, 1);
+        // 3D beyond the cache: fused rows and Y pass in turn over zc planes
+        const long long zc = fused && ny > 1 && ny <= kMaxFused
+                                 ? cache_planes(nz, ny * pitch * (long long)P->elem)
+                                 : nz;
+        rc = axis2(ny, Geo{zc, pitch * ny, cols, 1, pitch}, 1);
+        if (!rc && zc < nz) {
+            for (Pass &ps : P->passes) {
+                ps.group = 1;
+                ps.reps = nz / zc;
+                ps.rep_in = ps.rep_out = zc * ny * pitch;
+            }
+            P->passes[0].rep_in = zc * ny * m;
+        }
         if (!rc) rc = axis2(nz, Geo{ny, pitch, cols, 1, pitch * ny}, 2);
         if (!rc && cur != 1) rc = TOPE_ERROR_UNSUPPORTED;
         if (!rc && P->real_pack) {
