@@ -106,6 +106,13 @@ struct PlanImpl {
     bool pair_tiles = false;  // a pass moves complex64 column pairs (16-byte aligned arrays)
     int final_buf = 0;
     std::vector<Pass> passes;
+    // final_buf == 1: how callers' arrays, which must hold the result, run.
+    // Either the in-place pass alt_pass writes the other buffer and the passes
+    // after it work with exchanged buffers (while `alternate` is set), or
+    // ptr_passes is a schedule of its own; both end in buffer 0
+    int alt_pass = -1;
+    bool alternate = false;
+    std::vector<Pass> ptr_passes;
     std::vector<void *> allocs;
     std::map<std::pair<int, int>, void *> stage_tw;  // (n, e + 64 * prec) -> table
     struct AxisTw {
@@ -556,7 +563,7 @@ class Planner {
         if (n == 1) return TOPE_SUCCESS;
         if (n <= kMaxFused) return add_pass((int)n, g, g, *cur, *cur, 1, 0, 0, nullptr, nullptr, 0, 0, 0, 0, axis_id);
         if (n > kMaxLen) return TOPE_ERROR_INVALID_SIZE;
-        if (n > kMaxAxis) return three_step(n, g, cur, axis_id);
+        if (n > two_pass_max) return three_step(n, g, cur, axis_id);
         // four-step: i = n1 + N1*n2.  Step 1 transforms n2 (length N2, stride
         // N1*is) per (line, n1), multiplying output k2 by W_n^{n1*k2}, into
         // the other buffer (in place when `flip`); step 2 transforms n1
@@ -979,6 +986,8 @@ class Planner {
     // the two halves of each 128-byte line).  The real-input plans keep
     // each axis's data where it started.
     bool flip = false;
+    // a power-of-two axis runs two passes up to here, three above
+    long long two_pass_max = kMaxAxis;
 
    private:
     PlanImpl *P;
@@ -1039,8 +1048,9 @@ int launch_pass(PlanImpl *P, size_t i, hipStream_t s, int dir, long long rep0, l
     if (ps.kind == PASS_DONE) return TOPE_SUCCESS;
     const int sign = ((ps.fixed_dir >= 0 ? ps.fixed_dir : dir) == FORWARD) ? -1 : 1;
     const double sc = (dir == INVERSE) ? 1.0 / (double)P->norm : 1.0;
-    const char *ib = static_cast<const char *>(P->buf[ps.in_buf]);
-    char *ob = static_cast<char *>(P->buf[ps.out_buf]);
+    const int alt_in = P->alternate && (int)i > P->alt_pass, alt_out = P->alternate && (int)i >= P->alt_pass;
+    const char *ib = static_cast<const char *>(P->buf[ps.in_buf ^ alt_in]);
+    char *ob = static_cast<char *>(P->buf[ps.out_buf ^ alt_out]);
     const long long eb = (long long)P->elem;
     if (rep1 < 0) rep1 = ps.reps;
     if (ps.kind == PASS_AXIS) {
@@ -1168,7 +1178,7 @@ int enqueue(PlanImpl *P, hipStream_t s, int dir)
             P->pending.push_back({(int)i, {e0, e1}});
         }
     }
-    if (P->final_buf == 1) std::swap(P->buf[0], P->buf[1]);
+    if (P->final_buf == 1 && !P->alternate) std::swap(P->buf[0], P->buf[1]);
     return TOPE_SUCCESS;
 }
 
@@ -1397,6 +1407,30 @@ int build_plan(struct topeFFT *f, int shape, long long nx, long long ny, long lo
             break;
         }
     P->final_buf = cur;
+    if (cur == 1) {
+        for (size_t i = 0; i < P->passes.size() && P->alt_pass < 0; ++i)
+            if (P->passes[i].kind == PASS_AXIS && P->passes[i].in_buf == P->passes[i].out_buf) P->alt_pass = (int)i;
+        // Out of place, the four-step's narrow tiles write 64-byte segments
+        // of two arrays: once those outgrow the cache, three passes of
+        // short transforms in wide tiles take less time (1D FP64, forward +
+        // inverse: 2^24 645 us against 700; 2^23 311 against 315, 2^22 165
+        // against 146)
+        if ((shape == 1 || shape == SHAPE_BATCH) && mode == MP_VALU && is_pow2(nx) && nx <= kMaxAxis &&
+            nx * (long long)P->elem >= kCacheBytes) {
+            std::vector<Pass> own;
+            own.swap(P->passes);
+            Planner pc(P, s);
+            pc.two_pass_max = nx - 1;
+            int c = 0;
+            rc = pc.axis(nx, Geo{1, 0, shape == 1 ? 1 : ny, nx, 1}, &c, 0);
+            if (!rc && c == 0) {
+                P->ptr_passes.swap(P->passes);
+                P->ptr_passes.back().last = true;
+            }
+            P->passes.swap(own);
+            if (rc) return fail(rc);
+        }
+    }
     bool need_scratch = false;
     for (const Pass &ps : P->passes)
         if (ps.in_buf == 1 || ps.out_buf == 1) need_scratch = true;
@@ -2367,12 +2401,29 @@ void topePlanExecPtr(struct topeFFT *f, void *plan_impl, void *data, int dir)
         f->error = TOPE_ERROR_INVALID_ARG;
         return;
     }
-    // run the plan's passes with the caller's array in place of its own;
-    // schedules that end in the scratch buffer copy the result back
+    // run the plan's passes with the caller's array in place of its own.
+    // Where the plan's own data would end in its second buffer, one in-place
+    // pass writes that buffer instead (or another schedule runs), so the
+    // result ends in the caller's array; only a schedule without such a pass
+    // (short DFTs) copies it back.  Forward + inverse, 1D FP64: 2^13 21.4 ->
+    // 16.5 us, 2^16 22.6 -> 16.5 us, 2^20 64 -> 41 us, 2^24 882 -> 645 us
     void *own0 = P->buf[0], *own1 = P->buf[1];
     P->buf[0] = data;
+    const int final_buf = P->final_buf;
+    const bool own_list = !P->ptr_passes.empty();
+    P->alternate = !own_list && P->alt_pass >= 0;
+    if (own_list) {
+        P->passes.swap(P->ptr_passes);
+        P->final_buf = 0;
+    }
     int rc = enqueue(P, fw->stream, dir);
-    if (!rc && P->final_buf == 1)
+    const bool copy = P->final_buf == 1 && !P->alternate;
+    P->alternate = false;
+    if (own_list) {
+        P->passes.swap(P->ptr_passes);
+        P->final_buf = final_buf;
+    }
+    if (!rc && copy)
         rc = map_err(hipMemcpyAsync(data, P->buf[0], P->bytes, hipMemcpyDeviceToDevice, fw->stream));
     P->buf[0] = own0;
     P->buf[1] = own1;

@@ -39,8 +39,9 @@ namespace tope {
 constexpr int CT3_TW = 128 + 128;
 
 // Four-step post-twiddle factors of a tile (POST): for each column t of
-// base b_t, W^{b_t g} (g < 16), W^{16 b_t w} (w < 16) and W^{256 b_t}.
-constexpr int CT3_PT = 4 * 16 + 4 * 16 + 4;
+// base b_t, W^{b_t g} (g < 16), W^{16 b_t w} (w < 16), W^{256 b_t} and
+// W^{1024 b_t}.
+constexpr int CT3_PT = 4 * 16 + 4 * 16 + 4 + 4;
 
 template <typename R, bool POST = false>
 struct Ct3Lds {
@@ -109,9 +110,11 @@ __global__ void __launch_bounds__(1024) ct3_kernel(const cpx<R> *in, cpx<R> *out
     cpx<R> *ptl = ltw + CT3_TW;
     if constexpr (POST) {
         if (tid < CT3_PT) {
-            const int ct = tid < 128 ? (tid >> 4) & 3 : tid - 128;
+            const int ct = tid < 128 ? (tid >> 4) & 3 : tid & 3;
             const long long bt = o * a.pt_o + (long long)(c0 + ct) * a.pt_c;
-            const long long x = tid < 64 ? bt * (tid & 15) : tid < 128 ? bt * 16 * (tid & 15) : bt * 256;
+            const long long x = tid < 64    ? bt * (tid & 15)
+                                : tid < 128 ? bt * 16 * (tid & 15)
+                                            : bt * (tid < 132 ? 256 : 1024);
             ptl[tid] = pt_lookup(x, a.pt_lo, a.pt_hi, a.pt_n, a.pt_shift);
         }
     }
@@ -202,7 +205,7 @@ __global__ void __launch_bounds__(1024) ct3_kernel(const cpx<R> *in, cpx<R> *out
     if (!valid) return;
     // output rows k = g + 16 w + 256 e
     if constexpr (POST)  // W^{b k}, k = g + 16 w + 256 e: W^{b g} W^{16 b w} (W^{256 b})^e
-        pt_chain<SIGN>(v, cmul(ptl[16 * t + g], ptl[64 + 16 * t + w]), ptl[128 + t]);
+        pt_chain<SIGN>(v, cmul(ptl[16 * t + g], ptl[64 + 16 * t + w]), ptl[128 + t], ptl[132 + t]);
     if (a.scale != R(1)) {
 #pragma unroll
         for (int e = 0; e < 16; ++e) v[e] = scale(v[e], a.scale);

@@ -224,36 +224,40 @@ __device__ __forceinline__ cpx<R> pt_lookup(long long x, const cpx<R> *pt_lo, co
     return cmul(pt_lo[x & ((1LL << pt_shift) - 1)], pt_hi[x >> pt_shift]);
 }
 
-// v[e] *= w s^e: a chain of products of the step s (relative error ~E ulp
-// in FP64).
+// v[e] *= w s^e, with s4 = s^4 a value of its own: at most three factors s
+// and three factors s4 to an output, so the steps' own rounding errors enter
+// three times each, not up to 15 times as in a single chain of s.
 template <int SIGN, typename R, int E>
-__device__ __forceinline__ void pt_chain(cpx<R> (&v)[E], cpx<R> w, cpx<R> s)
+__device__ __forceinline__ void pt_chain(cpx<R> (&v)[E], cpx<R> w, cpx<R> s, cpx<R> s4)
 {
 #pragma unroll
-    for (int e = 0; e < E; ++e) {
-        if (e) w = cmul(w, s);
-        v[e] = twmul<SIGN>(v[e], w);
+    for (int e = 0; e < E; e += 4) {
+        if (e) w = cmul(w, s4);
+        cpx<R> u = w;
+#pragma unroll
+        for (int k = e; k < (e + 4 < E ? e + 4 : E); ++k) {
+            if (k > e) u = cmul(u, s);
+            v[k] = twmul<SIGN>(v[k], u);
+        }
     }
 }
 
 // Four-step post-twiddle of one thread's outputs k = p + P e (e < E) of a
 // line with twiddle base b: v[e] *= W_{pt_n}^{b k}.  W^{b (p + P e)} is
-// W^{b p} (W^{b P})^e: a fresh table value every RS outputs, products of
-// the step W^{b P} in between (FP64: one chain of E - 1 products, relative
-// error ~E ulp; FP32: fresh every 4 outputs); b k < 2^63.
+// W^{b p} (W^{b P})^e: products of the steps W^{b P} and W^{4 b P} (FP64), or
+// in FP32 a fresh table value every 4 outputs; b k < 2^63.
 template <int SIGN, typename R, int E>
 __device__ __forceinline__ void post_twiddle(cpx<R> (&v)[E], long long b, long long p, long long P,
                                              const cpx<R> *pt_lo, const cpx<R> *pt_hi, long long pt_n, int pt_shift)
 {
-    constexpr int RS = sizeof(R) == 8 ? E : 4;
-    if constexpr (RS == E) {
-        pt_chain<SIGN>(v, pt_lookup(b * p, pt_lo, pt_hi, pt_n, pt_shift), pt_lookup(b * P, pt_lo, pt_hi, pt_n, pt_shift));
+    const cpx<R> s = pt_lookup(b * P, pt_lo, pt_hi, pt_n, pt_shift);
+    cpx<R> w = pt_lookup(b * p, pt_lo, pt_hi, pt_n, pt_shift);
+    if constexpr (sizeof(R) == 8) {
+        pt_chain<SIGN>(v, w, s, E > 4 ? pt_lookup(4 * b * P, pt_lo, pt_hi, pt_n, pt_shift) : s);
     } else {
-        const cpx<R> s = pt_lookup(b * P, pt_lo, pt_hi, pt_n, pt_shift);
-        cpx<R> w = pt_lookup(b * p, pt_lo, pt_hi, pt_n, pt_shift);
 #pragma unroll
         for (int e = 0; e < E; ++e) {
-            if (e) w = (e % RS == 0) ? pt_lookup(b * (p + P * e), pt_lo, pt_hi, pt_n, pt_shift) : cmul(w, s);
+            if (e) w = (e % 4 == 0) ? pt_lookup(b * (p + P * e), pt_lo, pt_hi, pt_n, pt_shift) : cmul(w, s);
             v[e] = twmul<SIGN>(v[e], w);
         }
     }
