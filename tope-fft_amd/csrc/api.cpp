@@ -17,6 +17,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <map>
+#include <mutex>
 #include <new>
 #include <string>
 #include <utility>
@@ -47,7 +48,48 @@ struct FrameworkImpl {
     hipStream_t own = nullptr;     // the framework's own stream (stream unless a caller's is set)
     int live_plans = 0;
     EventPair last;  // last exec's device time (profileThis)
+    hipEvent_t copied = nullptr;  // behind the download of the last small exec
+    bool stage_ref = false;       // this framework holds a reference to the staging buffer
 };
+
+// Pinned staging buffer for the downloads of small synchronous execs, one for
+// the process: taken by the first exec that wants it, given back with the last
+// framework that used it.  An exec holds it (a try_lock) from its launch
+// until it has copied the result out; one that finds it held downloads by
+// itself.
+constexpr size_t kStageBytes = 256 << 10;
+struct Staging {
+    std::mutex mu;    // buf and users
+    std::mutex busy;  // held by the exec that uses the buffer
+    void *buf = nullptr;
+    int users = 0;
+} g_stage;
+
+void *stage_take(FrameworkImpl *fw)
+{
+    std::lock_guard<std::mutex> lk(g_stage.mu);
+    if (!fw->stage_ref) {
+        if (!g_stage.buf && hipHostMalloc(&g_stage.buf, kStageBytes, hipHostMallocPortable) != hipSuccess) {
+            g_stage.buf = nullptr;
+            (void)hipGetLastError();
+            return nullptr;
+        }
+        fw->stage_ref = true;
+        ++g_stage.users;
+    }
+    return g_stage.buf;
+}
+
+void stage_release(FrameworkImpl *fw)
+{
+    std::lock_guard<std::mutex> lk(g_stage.mu);
+    if (!fw->stage_ref) return;
+    fw->stage_ref = false;
+    if (--g_stage.users == 0) {
+        (void)hipHostFree(g_stage.buf);
+        g_stage.buf = nullptr;
+    }
+}
 
 enum PassKind {
     PASS_AXIS = 0,
@@ -1659,10 +1701,42 @@ void release_framework(struct topeFFT *f)
     }
     if (fw->last.start) (void)hipEventDestroy(fw->last.start);
     if (fw->last.stop) (void)hipEventDestroy(fw->last.stop);
+    if (fw->copied) (void)hipEventDestroy(fw->copied);
+    stage_release(fw);
     delete fw;
     f->impl = nullptr;
     f->stream = nullptr;
     f->event = nullptr;
+}
+
+double elapsed_ns(hipEvent_t a, hipEvent_t b)
+{
+    float ms = 0;
+    return hipEventElapsedTime(&ms, a, b) == hipSuccess ? (double)ms * 1e6 : 0.0;
+}
+
+// Exec of a transform of at most kStageBytes into host memory: transform, a
+// copy kernel into the pinned staging buffer, one wait for both, then the copy
+// into d.  The general path waits for the transform, then for a copy that
+// the runtime stages itself, and makes two events for each call.
+// @@HFIG@@
+int exec_staged(FrameworkImpl *fw, PlanImpl *P, void *stage, void *d, int dir, tope_ulong *kern_ns, tope_ulong *mem_ns)
+{
+    hipStream_t s = fw->stream;
+    hipError_t err = ensure_event(&fw->copied);
+    if (err == hipSuccess) err = time_start(fw->last, s, false);
+    if (err != hipSuccess) return map_err(err);
+    const int rc = enqueue(P, s, dir);
+    if (rc) return rc;
+    err = time_stop(fw->last, s, nullptr);
+    if (err == hipSuccess) err = copy_out(P->buf[0], stage, P->bytes, s);
+    if (err == hipSuccess) err = hipEventRecord(fw->copied, s);
+    if (err == hipSuccess) err = hipEventSynchronize(fw->copied);
+    if (err != hipSuccess) return map_err(err);
+    std::memcpy(d, stage, P->bytes);
+    *kern_ns += (tope_ulong)elapsed_ns(fw->last.start, fw->last.stop);
+    *mem_ns += (tope_ulong)elapsed_ns(fw->last.stop, fw->copied);
+    return TOPE_SUCCESS;
 }
 
 // Exec with the reference's semantics: transform, then blocking copy of the
@@ -1672,6 +1746,12 @@ int exec_host(struct topeFFT *f, PlanImpl *P, void *d, int dir, tope_ulong *kern
     FrameworkImpl *fw = fw_of(f);
     if (!fw || P->fw != fw) return TOPE_ERROR_NOT_INITIALIZED;
     if (!d) return TOPE_ERROR_INVALID_ARG;
+    if (P->bytes <= kStageBytes && !P->timing) {
+        if (void *stage = stage_take(fw)) {
+            std::unique_lock<std::mutex> hold(g_stage.busy, std::try_to_lock);
+            if (hold.owns_lock()) return exec_staged(fw, P, stage, d, dir, kern_ns, mem_ns);
+        }
+    }
     hipStream_t s = fw->stream;
     hipError_t err = time_start(fw->last, s);
     if (err != hipSuccess) return map_err(err);

@@ -61,6 +61,9 @@ hipError_t gen_power_table(void *out, int prec, long long M, long long mult, lon
 hipError_t launch_naive_dft(int prec, const void *in, void *out, const void *roots, long long n, int sign,
                             double scale, hipStream_t s);
 
+// `bytes` (a multiple of 8) from device to device-visible memory by a kernel.
+hipError_t copy_out(const void *in, void *out, size_t bytes, hipStream_t s);
+
 // Mixed-precision MFMA rows (mfma_kernel.hpp).
 struct MfmaArgs;
 hipError_t gen_mfma_constants(void *out, hipStream_t s);

@@ -163,4 +163,21 @@ hipError_t launch_naive_dft(int prec, const void *in, void *out, const void *roo
     return hipGetLastError();
 }
 
+// One 8-byte word a thread: the small results that go to pinned host memory
+// (a store instruction of a wave is 512 contiguous bytes on the bus).
+__global__ void copy_out_kernel(const unsigned long long *in, unsigned long long *out, unsigned n)
+{
+    const unsigned i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) out[i] = in[i];
+}
+
+hipError_t copy_out(const void *in, void *out, size_t bytes, hipStream_t s)
+{
+    const unsigned n = (unsigned)(bytes / 8);
+    if (bytes % 8 || n < 1) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(copy_out_kernel, dim3((n + 255) / 256), dim3(256), 0, s,
+                       static_cast<const unsigned long long *>(in), static_cast<unsigned long long *>(out), n);
+    return hipGetLastError();
+}
+
 }  // namespace tope
