@@ -36,6 +36,7 @@ namespace {
 constexpr int kMaxFused = 4096;          // longest axis one pass holds on chip
 constexpr long long kMaxAxis = 1LL << 24;  // four-step limit (4096 x 4096)
 constexpr long long kMaxLen = 1LL << 30;   // three-pass limit of a power-of-two axis here (16 GiB FP64)
+constexpr long long kCacheBytes = 256LL << 20;  // Infinity Cache
 constexpr long long kChirpMin = 64;        // longer non-power-of-two 1D lengths use Bluestein
 
 struct EventPair {
@@ -118,6 +119,9 @@ struct Pass {
     int group = 0;  // != 0: neighbours of one group run their launches in turn (chunks)
     long long base = 0;                           // element offset of the pass's geometry in both buffers
     bool last = false;                            // receives the inverse 1/N scale
+    int stream = 0;             // STREAM_LOAD, STREAM_STORE of an axis pass
+    bool stream_moved = false;  // STREAM_LOAD too when the pass writes another buffer than it reads
+    AxisLaunchFn stream_fn = nullptr;  // launches the pass's streaming form
     long long dft_n = 0;
     const void *dft_roots = nullptr;
     const void *real_w = nullptr;  // PASS_REAL: W_n^k, k = 0..m (FP64)
@@ -1094,10 +1098,17 @@ int launch_pass(PlanImpl *P, size_t i, hipStream_t s, int dir, long long rep0, l
     const char *ib = static_cast<const char *>(P->buf[ps.in_buf ^ alt_in]);
     char *ob = static_cast<char *>(P->buf[ps.out_buf ^ alt_out]);
     const long long eb = (long long)P->elem;
+    const int stream = ps.stream | (ps.stream_moved && ib != ob ? STREAM_LOAD : 0);
     if (rep1 < 0) rep1 = ps.reps;
+    AxisLaunchFn launch = nullptr;
+    if (ps.kind == PASS_AXIS) {
+        launch = ps.var->fn;
+        if (stream && ps.stream_fn) launch = ps.stream_fn;
+    }
     if (ps.kind == PASS_AXIS) {
         if (ps.var->prec == PREC_F64) {
             AxisArgs<double> a = ps.a;
+            a.stream = stream;
             a.scale = ps.last ? sc : 1.0;
             a.in_elems -= ps.base;
             a.out_elems -= ps.base;
@@ -1105,11 +1116,12 @@ int launch_pass(PlanImpl *P, size_t i, hipStream_t s, int dir, long long rep0, l
             for (long long r = rep0; r < rep1; ++r) {
                 a.in_elems = ie - r * ps.rep_in;
                 a.out_elems = oe - r * ps.rep_out;
-                ps.var->fn(ib + (ps.base + r * ps.rep_in) * eb, ob + (ps.base + r * ps.rep_out) * eb, &a, ps.grid, s,
+                launch(ib + (ps.base + r * ps.rep_in) * eb, ob + (ps.base + r * ps.rep_out) * eb, &a, ps.grid, s,
                            sign);
             }
         } else {
             AxisArgs<float> a = ps.a32;
+            a.stream = stream;
             a.scale = ps.last ? (float)sc : 1.0f;
             a.in_elems -= ps.base;
             a.out_elems -= ps.base;
@@ -1117,7 +1129,7 @@ int launch_pass(PlanImpl *P, size_t i, hipStream_t s, int dir, long long rep0, l
             for (long long r = rep0; r < rep1; ++r) {
                 a.in_elems = ie - r * ps.rep_in;
                 a.out_elems = oe - r * ps.rep_out;
-                ps.var->fn(ib + (ps.base + r * ps.rep_in) * eb, ob + (ps.base + r * ps.rep_out) * eb, &a, ps.grid, s,
+                launch(ib + (ps.base + r * ps.rep_in) * eb, ob + (ps.base + r * ps.rep_out) * eb, &a, ps.grid, s,
                            sign);
             }
         }
@@ -1235,6 +1247,42 @@ PlanImpl *impl_of(void *p) { return static_cast<PlanImpl *>(p); }
 
 enum { SHAPE_BATCH = 4 };
 
+// Which passes of a plan's list stream through L2 (axis_kernel.hpp): only
+// those of plans whose arrays outgrow the 256 MB Infinity Cache twice over.
+// Streamed lines skip that cache too, and a smaller array is found there
+// again by the next transform or the caller's next kernel: FP64 4096 x 4096
+// (256 MiB) transformed over and over on one array 67 us, streamed 98 (several
+// arrays in turn: 109, streamed 96).  From 512 MiB on both are faster streamed.
+// Figures: one transform, over and over on one array.
+void set_streaming(PlanImpl *P, std::vector<Pass> &L)
+{
+    if (L.empty()) return;
+    bool two = false;
+    for (const Pass &ps : L) two = two || ps.in_buf != ps.out_buf;
+    if ((long long)P->bytes * (two ? 2 : 1) < 2 * kCacheBytes) return;
+    int cnt = 0;
+    const AxisVariant *base = axis_variants(&cnt), *sv = axis_variants_stream(&cnt);
+    for (Pass &ps : L)  // (64-bit instantiations keep their own launch)
+        if (ps.kind == PASS_AXIS && ps.var >= base && ps.var < base + cnt) ps.stream_fn = sv[ps.var - base].fn;
+    Pass &first = L.front(), &last = L.back();
+    if (L.size() == 1) {
+        // rows in one pass (batches), if a wave's instruction covers whole
+        // lines: FP64 8192 x 4096 217 -> 197 us, complex64 16384 x 4096 196 -> 175;
+        // 64-point rows (64-byte pieces) lose a third
+        if (first.kind == PASS_AXIS && !first.var->cfast && first.stream_fn) first.stream = STREAM_LOAD | STREAM_STORE;
+        return;
+    }
+    // a first pass that moves the data reads it for the last time; in place it
+    // would write back what it dropped (2D 4096^2 190 -> 223 us).  A last pass that
+    // moves it, or whose tiles write whole lines, leaves what nobody reads:
+    // 1D 2^24 (callers' arrays) 315 -> 251 us with both, complex64 512^3
+    // 1060 -> 1030 us
+    if (first.kind == PASS_AXIS && first.stream_fn && first.a.pt_n) first.stream_moved = true;
+    if (last.kind != PASS_AXIS || !last.stream_fn || !last.var->cfast) return;
+    if (last.in_buf != last.out_buf) last.stream = STREAM_STORE;
+    else if (last.var->tb * (long long)P->elem >= 128) last.stream = STREAM_LOAD | STREAM_STORE;
+}
+
 // Planes of a volume that the X and Y passes take at a time.  Beyond the 256
 // MB Infinity Cache the Y pass would read back from memory what the X pass
 // wrote; over chunks that fill the cache it finds part of it there: 512^3
@@ -1246,7 +1294,6 @@ enum { SHAPE_BATCH = 4 };
 // lose 7 % at 512 x 256 x 256, whose spectrum is just larger than the cache.
 // All planes at once below twice the cache, or when no divisor of nz gives
 // half of it.
-constexpr long long kCacheBytes = 256LL << 20;
 long long cache_planes(long long nz, long long plane_bytes)
 {
     if (nz * plane_bytes < 2 * kCacheBytes) return nz;
@@ -1473,6 +1520,8 @@ int build_plan(struct topeFFT *f, int shape, long long nx, long long ny, long lo
             if (rc) return fail(rc);
         }
     }
+    set_streaming(P, P->passes);
+    set_streaming(P, P->ptr_passes);
     bool need_scratch = false;
     for (const Pass &ps : P->passes)
         if (ps.in_buf == 1 || ps.out_buf == 1) need_scratch = true;

@@ -56,6 +56,15 @@ struct Sched {
     static constexpr int TWSIZE = twoff(NST);
 };
 
+// Data accesses of a pass that ask L2 to drop their lines first.  Stores: the
+// lines are written out while the pass runs instead of staying dirty in the
+// 32 MB of L2 until the kernel ends (a kernel boundary costs about 6 us of
+// write-back); loads: what is read for the last time makes room for the
+// stores.  Only where an instruction covers whole 128-byte lines, or the
+// lines go to a buffer that the pass does not read: elsewhere the two halves
+// of a line no longer meet in L2.
+constexpr int STREAM_LOAD = 1, STREAM_STORE = 2;
+
 // Kernel arguments (all strides in complex elements).
 template <typename R>
 struct AxisArgs {
@@ -75,6 +84,7 @@ struct AxisArgs {
     int xcd;    // 1: remap blocks so each XCD walks a contiguous range of tiles
     int rot;    // 0 <= rot < tiles: logical tile t of an outer index runs tile
                 // (t + rot) mod tiles (a partial last tile can go first)
+    int stream;  // STREAM_LOAD, STREAM_STORE: selects the streaming instantiation
     long long in_elems, out_elems;  // buffer sizes (bounds of the buffer resources)
     // DIF2 row passes: block-local transform t = 2q + h is row (tile*TB/2 + q)
     // shifted by h*pair elements; afterwards the two rows of each pair are
@@ -164,14 +174,17 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void *base, lo
 typedef unsigned int tope_u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int tope_u32x2 __attribute__((ext_vector_type(2)));
 
-template <typename R>
+// Cache policy of a load or store: CP_STREAM marks its lines first to leave L2.
+constexpr int CP_KEEP = 0, CP_STREAM = 2;
+
+template <typename R, int CP = CP_KEEP>
 __device__ __forceinline__ cpx<R> buf_load(__amdgpu_buffer_rsrc_t r, int voff, int soff)
 {
     if constexpr (sizeof(R) == 8) {
-        tope_u32x4 u = __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0);
+        tope_u32x4 u = __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, CP);
         return __builtin_bit_cast(cpx<R>, u);
     } else {
-        tope_u32x2 u = __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 0);
+        tope_u32x2 u = __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, CP);
         return __builtin_bit_cast(cpx<R>, u);
     }
 }
@@ -183,13 +196,13 @@ __device__ __forceinline__ cpx<R> buf_load(__amdgpu_buffer_rsrc_t r, int voff, i
 // VALU write issued right after the store has replaced the upper dwords of
 // the stored value in some lanes.  With an inline-constant soffset the
 // compiler inserts the wait state.
-template <typename R>
+template <typename R, int CP = CP_KEEP>
 __device__ __forceinline__ void buf_store(cpx<R> v, __amdgpu_buffer_rsrc_t r, int voff, int soff)
 {
     if constexpr (sizeof(R) == 8)
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(tope_u32x4, v), r, voff + soff, 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(tope_u32x4, v), r, voff + soff, 0, CP);
     else
-        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(tope_u32x2, v), r, voff, soff, 0);
+        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(tope_u32x2, v), r, voff, soff, CP);
 }
 
 // Table values read at a block's start and used after its data loads are
@@ -446,14 +459,15 @@ constexpr int axis_lds_bytes()
 }
 
 // One logical block (tile blk) of an axis pass: TB transforms.  POST applies
-// the four-step post-twiddle; the output scale is runtime-uniform.
+// the four-step post-twiddle; the output scale is runtime-uniform; ST holds
+// the pass's STREAM_ bits.
 //
 // Global accesses go through buffer resources based at the block's first
 // element: each thread keeps one 32-bit byte offset and the per-element
 // stride e*P*is*16 is a uniform (SGPR) offset, which keeps address
 // registers out of the way of the 4*E data registers.  Blocks whose
 // footprint exceeds 2^31 bytes run the BIG instantiation (64-bit pointers).
-template <typename R, int N, int E, int TB, bool CFAST, bool SPLIT, int SIGN, bool POST, bool BIG, bool DIF2>
+template <typename R, int N, int E, int TB, bool CFAST, bool SPLIT, int SIGN, bool POST, bool BIG, bool DIF2, int ST>
 __device__ __forceinline__ void axis_block(const cpx<R> *in, cpx<R> *out, const AxisArgs<R> &a, long long blk,
                                            unsigned char *lds)
 {
@@ -501,7 +515,8 @@ __device__ __forceinline__ void axis_block(const cpx<R> *in, cpx<R> *out, const 
         const int sstep = (int)((long long)P * a.in_is * CB);
         if (valid) {
 #pragma unroll
-            for (int e = 0; e < E; ++e) v[e] = buf_load<R>(rin, voff, e * sstep);
+            for (int e = 0; e < E; ++e)
+                v[e] = buf_load<R, (ST & STREAM_LOAD) ? CP_STREAM : CP_KEEP>(rin, voff, e * sstep);
         } else {
 #pragma unroll
             for (int e = 0; e < E; ++e) v[e] = cpx<R>{0, 0};
@@ -568,7 +583,8 @@ __device__ __forceinline__ void axis_block(const cpx<R> *in, cpx<R> *out, const 
         const int voff = (int)((tr * a.out_cs + hoff + (long long)p * a.out_is) * CB);
         const int sstep = (int)((long long)P * a.out_is * CB);
 #pragma unroll
-        for (int e = 0; e < E; ++e) buf_store<R>(v[e], rout, voff, e * sstep);
+        for (int e = 0; e < E; ++e)
+            buf_store<R, (ST & STREAM_STORE) ? CP_STREAM : CP_KEEP>(v[e], rout, voff, e * sstep);
     } else {
         cpx<R> *dst = out + o * a.out_os + (long long)c * a.out_cs + hoff;
 #pragma unroll
@@ -577,12 +593,13 @@ __device__ __forceinline__ void axis_block(const cpx<R> *in, cpx<R> *out, const 
 }
 
 // One launch = one axis pass, one workgroup per logical block.
-template <typename R, int N, int E, int TB, bool CFAST, bool SPLIT, int SIGN, bool POST, bool BIG, bool DIF2 = false>
+template <typename R, int N, int E, int TB, bool CFAST, bool SPLIT, int SIGN, bool POST, bool BIG, bool DIF2 = false,
+          int ST = 0>
 __global__ void __launch_bounds__(TB *(N / E))
 axis_kernel(const cpx<R> *in, cpx<R> *out, const AxisArgs<R> a)
 {
     __shared__ __align__(16) unsigned char lds[axis_lds_bytes<R, N, E, TB, CFAST, SPLIT, DIF2>()];
-    axis_block<R, N, E, TB, CFAST, SPLIT, SIGN, POST, BIG, DIF2>(in, out, a, xcd_block(a.xcd), lds);
+    axis_block<R, N, E, TB, CFAST, SPLIT, SIGN, POST, BIG, DIF2, ST>(in, out, a, xcd_block(a.xcd), lds);
 }
 
 }  // namespace tope

@@ -37,6 +37,9 @@ struct AxisVariant {
 const AxisVariant *axis_variants(int *count);
 // Same list, same order, compiled with 64-bit addressing.
 const AxisVariant *axis_variants_big(int *count);
+// Same list, same order: launches of AxisArgs::stream passes, fn null where
+// a variant has none.
+const AxisVariant *axis_variants_stream(int *count);
 
 // Runtime mirror of Sched<N, E> (the device derives the same layout at
 // compile time; api.cpp checks that both agree for every variant).

@@ -40,6 +40,43 @@ static void launch_axis_t(const void *in, void *out, const void *args, unsigned 
                            i, o, a);
 }
 
+#ifdef TOPE_AXIS_STREAM
+// Streaming instantiations: rows of one-pass plans (both), a moving first pass
+// (POST: loads) or last pass (stores), a last pass in place whose tiles write
+// whole 128-byte lines (both); nullptr where no plan of 512 MiB comes.
+template <typename R, int N, int E, int TB, bool CFAST, bool SPLIT>
+static void launch_stream_t(const void *in, void *out, const void *args, unsigned grid, hipStream_t s, int sign)
+{
+    const AxisArgs<R> &a = *static_cast<const AxisArgs<R> *>(args);
+    const cpx<R> *i = static_cast<const cpx<R> *>(in);
+    cpx<R> *o = static_cast<cpx<R> *>(out);
+    const dim3 g(grid), b(TB * (N / E));
+    constexpr int BOTH = STREAM_LOAD | STREAM_STORE;
+#define TOPE_STREAM(POST, ST)                                                                                       \
+    do {                                                                                                            \
+        if (sign < 0)                                                                                               \
+            hipLaunchKernelGGL((axis_kernel<R, N, E, TB, CFAST, SPLIT, -1, POST, false, false, ST>), g, b, 0, s, i, o, a); \
+        else                                                                                                        \
+            hipLaunchKernelGGL((axis_kernel<R, N, E, TB, CFAST, SPLIT, 1, POST, false, false, ST>), g, b, 0, s, i, o, a);  \
+    } while (0)
+    if constexpr (!CFAST) {
+        TOPE_STREAM(false, BOTH);
+    } else if (a.pt_n) {
+        TOPE_STREAM(true, STREAM_LOAD);
+    } else if (a.stream == STREAM_STORE) {
+        TOPE_STREAM(false, STREAM_STORE);
+    } else {
+        TOPE_STREAM(false, BOTH);
+    }
+}
+template <typename R, int N, int E, int TB, bool CF, bool SP, bool DF>
+constexpr AxisLaunchFn stream_launch()
+{
+    if constexpr (!DF && N >= 128 && (CF ? TB >= 4 : N / E * sizeof(cpx<R>) >= 128)) return &launch_stream_t<R, N, E, TB, CF, SP>;
+    else return nullptr;
+}
+#endif
+
 // Even/odd-split column tiles (dit2_kernel): NT = TB * (N/2) / E threads.
 template <typename R, int N, int E, int TB, bool SPLIT, bool BIG>
 static void launch_dit2_t(const void *in, void *out, const void *args, unsigned grid, hipStream_t s, int sign)
@@ -94,7 +131,12 @@ static void launch_ct3p_t(const void *in, void *out, const void *args, unsigned 
     }
 }
 
-#ifdef TOPE_AXIS_BIG
+#ifdef TOPE_AXIS_STREAM
+#define TOPE_LAUNCH_CT3P nullptr
+#define TOPE_LAUNCH_CT3(R) nullptr
+#define TOPE_LAUNCH(R, N, E, TB, CF, SP, DF) stream_launch<R, N, E, TB, CF, SP, DF>()
+#define TOPE_LAUNCH_DIT2(R, N, E, TB, SP) nullptr
+#elif defined(TOPE_AXIS_BIG)
 #define TOPE_LAUNCH_CT3P &launch_ct3p_t<true>
 #define TOPE_LAUNCH_CT3(R) &launch_ct3_t<R, true>
 #define TOPE_LAUNCH(R, N, E, TB, CF, SP, DF) &launch_axis_t<R, N, E, TB, CF, SP, true, DF>
@@ -183,9 +225,12 @@ static const AxisVariant kVariants[] = {ROWS(double), COLS(double), DIF2ROWS(dou
                                         VARH(float, 4096, 16, 8, false), VAR(float, 4096, 32, 8, true, true),
                                         VARC(double), VARCP};
 
-// The same list is compiled twice: normally (32-bit buffer offsets) and with
-// TOPE_AXIS_BIG (64-bit pointers) for blocks spanning more than 2^31 bytes.
-#ifdef TOPE_AXIS_BIG
+// The same list is compiled three times: normally (32-bit buffer offsets), with
+// TOPE_AXIS_BIG (64-bit pointers) for blocks spanning more than 2^31 bytes, and
+// with TOPE_AXIS_STREAM (32-bit offsets, streaming accesses).
+#ifdef TOPE_AXIS_STREAM
+const AxisVariant *axis_variants_stream(int *count)
+#elif defined(TOPE_AXIS_BIG)
 const AxisVariant *axis_variants_big(int *count)
 #else
 const AxisVariant *axis_variants(int *count)

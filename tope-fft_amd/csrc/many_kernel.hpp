@@ -56,7 +56,7 @@ __device__ __forceinline__ ManyTask many_task(const A &a, int k)
     return tk;
 }
 
-template <typename R, int N, int E, int SIGN, int NT>
+template <typename R, int N, int E, int SIGN, int NT, bool STREAM>
 __device__ __forceinline__ void many_rows(const cpx<R> *in, cpx<R> *out, const ManyArgs<R> &a, int k, void *lds)
 {
     constexpr int P = N / E;
@@ -84,7 +84,10 @@ __device__ __forceinline__ void many_rows(const cpx<R> *in, cpx<R> *out, const M
     const R sc = SIGN > 0 ? (R)(1.0 / N) : (R)1;  // INVERSE: 1/n, a power of two (exact)
     if (valid) {
 #pragma unroll
-        for (int e = 0; e < E; ++e) buf_store<R>(scale(v[e], sc), wsrc, voff, e * sstep);
+        for (int e = 0; e < E; ++e) {
+            // only stores that cover whole 128-byte lines stream
+            buf_store<R, (STREAM && P * CB >= 128) ? CP_STREAM : CP_KEEP>(scale(v[e], sc), wsrc, voff, e * sstep);
+        }
     }
 }
 
@@ -94,25 +97,25 @@ constexpr int many_lds_bytes() { return NT / 16 * 17 * 16 * (int)sizeof(R); }
 
 // Dispatch one task of class L to its schedule (E = 8 only where n/8 threads
 // fit the block).
-template <typename R, int L, int SIGN, int NT>
+template <typename R, int L, int SIGN, int NT, bool STREAM>
 __device__ __forceinline__ void many_class(const cpx<R> *in, cpx<R> *out, const ManyArgs<R> &a, int k, void *lds,
                                            bool e8)
 {
     constexpr int N = 1 << L;
     if constexpr (N >= 8 && N / 8 <= NT) {
         if (e8) {
-            many_rows<R, N, 8, SIGN, NT>(in, out, a, k, lds);
+            many_rows<R, N, 8, SIGN, NT, STREAM>(in, out, a, k, lds);
             return;
         }
     }
-    if constexpr ((N < 16 ? 1 : N / 16) <= NT) many_rows<R, N, (N < 16 ? N : 16), SIGN, NT>(in, out, a, k, lds);
+    if constexpr ((N < 16 ? 1 : N / 16) <= NT) many_rows<R, N, (N < 16 ? N : 16), SIGN, NT, STREAM>(in, out, a, k, lds);
 }
 
 // Tasks of one class: this block takes global task indices b, b + G, ...
 // that fall in [seg0[L], seg1[L]) -- the same round-robin deal as one loop
 // over the whole list, but each loop body holds one class's code, which keeps
 // the register allocation of the 1024-thread block free of spills.
-template <typename R, int L, int SIGN, int NT>
+template <typename R, int L, int SIGN, int NT, bool STREAM>
 __device__ __forceinline__ void many_segment(const cpx<R> *in, cpx<R> *out, const ManyArgs<R> &a, void *lds)
 {
     const int s0 = a.seg0[L], s1 = a.seg1[L];
@@ -121,7 +124,7 @@ __device__ __forceinline__ void many_segment(const cpx<R> *in, cpx<R> *out, cons
     int task = s0 + ((b - s0) % G + G) % G;
     const bool e8 = a.sched[L] != 0;
     for (; task < s1; task += G) {
-        many_class<R, L, SIGN, NT>(in, out, a, task - s0, lds, e8);
+        many_class<R, L, SIGN, NT, STREAM>(in, out, a, task - s0, lds, e8);
         __syncthreads();  // the next task reuses the LDS
     }
 }
@@ -131,25 +134,26 @@ __device__ __forceinline__ void many_segment(const cpx<R> *in, cpx<R> *out, cons
 // points (the last for its radix-8 schedule, 512 threads per transform) at
 // 1024 threads; every class up to 4096 points at 256, capped at 128 VGPRs
 // so four blocks share a CU.
-template <typename R, int SIGN, int NT>
+// STREAM: the stores stream through L2 (axis_kernel.hpp).
+template <typename R, int SIGN, int NT, bool STREAM>
 __global__ void __launch_bounds__(NT, NT >= 1024 ? 1 : 4) many_kernel(const cpx<R> *in, cpx<R> *out,
                                                                      const ManyArgs<R> a)
 {
     __shared__ __align__(16) unsigned char lds[many_lds_bytes<R, NT>()];
     if constexpr (NT >= 1024) {
-        many_segment<R, 14, SIGN, NT>(in, out, a, lds);
-        many_segment<R, 13, SIGN, NT>(in, out, a, lds);
-        many_segment<R, 12, SIGN, NT>(in, out, a, lds);
+        many_segment<R, 14, SIGN, NT, STREAM>(in, out, a, lds);
+        many_segment<R, 13, SIGN, NT, STREAM>(in, out, a, lds);
+        many_segment<R, 12, SIGN, NT, STREAM>(in, out, a, lds);
     } else {
-        many_segment<R, 12, SIGN, NT>(in, out, a, lds);
-        many_segment<R, 11, SIGN, NT>(in, out, a, lds);
-        many_segment<R, 10, SIGN, NT>(in, out, a, lds);
-        many_segment<R, 9, SIGN, NT>(in, out, a, lds);
-        many_segment<R, 8, SIGN, NT>(in, out, a, lds);
-        many_segment<R, 7, SIGN, NT>(in, out, a, lds);
-        many_segment<R, 6, SIGN, NT>(in, out, a, lds);
-        many_segment<R, 5, SIGN, NT>(in, out, a, lds);
-        many_segment<R, 4, SIGN, NT>(in, out, a, lds);
+        many_segment<R, 12, SIGN, NT, STREAM>(in, out, a, lds);
+        many_segment<R, 11, SIGN, NT, STREAM>(in, out, a, lds);
+        many_segment<R, 10, SIGN, NT, STREAM>(in, out, a, lds);
+        many_segment<R, 9, SIGN, NT, STREAM>(in, out, a, lds);
+        many_segment<R, 8, SIGN, NT, STREAM>(in, out, a, lds);
+        many_segment<R, 7, SIGN, NT, STREAM>(in, out, a, lds);
+        many_segment<R, 6, SIGN, NT, STREAM>(in, out, a, lds);
+        many_segment<R, 5, SIGN, NT, STREAM>(in, out, a, lds);
+        many_segment<R, 4, SIGN, NT, STREAM>(in, out, a, lds);
     }
 }
 
