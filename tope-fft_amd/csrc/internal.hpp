@@ -115,6 +115,7 @@ struct MixedArgs {
     int cap;         // elements a thread can hold at the list's radices
     int twsize;      // entries of the stage table
     int nt, tb;      // threads and lines per block
+    int tbp;         // LDS slots between the elements of a strided line
     float inv_tb;
     double inv_C;
     const void *tw;  // stage table (gen_mixed_table), in the pass's precision

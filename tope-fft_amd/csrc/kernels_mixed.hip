@@ -104,14 +104,20 @@ void mixed_schedule(MixedArgs &a, int prec)
     // Tile: 256 threads, or as many more as a line (rows) or a 64-byte wide
     // tile (strided lines) needs.  Of the line counts that fit, the one whose
     // last wave of blocks leaves the least idle: a block costs its elements
-    // plus a fixed latency worth about 1000 more, and 16 waves (four per
-    // SIMD at 128 registers) or 160 KiB of LDS fill a CU.  Against the widest
-    // tile that fits: 100^3 67.8 -> 63.5 us, 200 x 180 x 150 212 -> 200 us,
+    // plus a fixed latency worth about 1000 more, and 16 waves (four per SIMD at
+    // 128 registers) or 160 KiB of LDS fill a CU.  Against the widest tile that
+    // fits: 100^3 67.8 -> 63.5 us, 200 x 180 x 150 212 -> 200 us,
     // 48 x 60 x 56 40.0 -> 33.3 us (a forward and an inverse transform).
+    // Strided lines take rows in segments of tb elements, and below 64 bytes
+    // each costs more than its bytes: 2400 x 2400 takes 182 us in segments of
+    // 64 bytes, 208 to 210 in 32 or 48 and 281 in 16 (its rows 88 of each).  A
+    // higher factor for 32 bytes loses where those tiles fill the chip better:
+    // 900 x 900 50.7 us in 32 bytes, 55.5 in 16.
     const int eb = prec == PREC_F64 ? 16 : 8;
     const bool col = a.is != 1 || a.ois != 1;
     const int want = col ? 64 / eb : 1;
     a.nt = 256;
+    a.tbp = 1;
     if (a.nst == 1) {
         a.tb = 256;
     } else {
@@ -120,15 +126,26 @@ void mixed_schedule(MixedArgs &a, int prec)
         double best = 0;
         for (int tb = most; tb >= 1; --tb) {
             if (tb != most && tb > want && tb % want) continue;  // whole 64-byte segments
-            const long long bytes = (col ? mixed_slots<true>(a.n, tb) : mixed_slots<false>(a.n, tb)) * (long long)eb;
+            // an odd distance between a line's elements spreads the first
+            // stage's writes over the banks; given up where the tile fits
+            // only without (3600 x 3600, two lines for one: 570 -> 420 us)
+            int tbp = tb | 1;
+            if (col && (long long)a.n * tbp * eb > MIXED_LDS) tbp = tb;
+            const long long bytes = (long long)eb * (col ? mixed_slots<true>(a.n, tb, tbp) : mixed_slots<false>(a.n, tb, tbp));
             if (bytes > MIXED_LDS) continue;
             const long long slots = 256 * std::min<long long>(MIXED_LDS / bytes, 1024 / a.nt);
             const long long blocks = (a.lines + tb - 1) / tb;
-            const double cost = (double)((blocks + slots - 1) / slots) * ((double)tb * a.n + 1000.0);
-            if (best == 0 || cost < best) best = cost, a.tb = tb;
+            const int seg = col ? tb * eb : 64;  // bytes of a row that a tile takes
+            const double mem = seg < 32 ? 1.9 : seg < 64 ? 1.2 : 1.0;
+            const double cost = (double)((blocks + slots - 1) / slots) * ((double)tb * a.n + 1000.0) * mem;
+            if (best == 0 || cost < best) best = cost, a.tb = tb, a.tbp = tbp;
         }
     }
-    if (a.tb > a.lines) a.tb = (int)a.lines;
+    if (a.tb > a.lines) {
+        a.tb = (int)a.lines;
+        a.tbp = a.tb | 1;
+        if (col && (long long)a.n * a.tbp * eb > MIXED_LDS) a.tbp = a.tb;
+    }
     a.inv_tb = 1.0f / (float)a.tb;
     a.inv_C = 1.0 / (double)a.C;
     a.inv_split = a.pt_split > 0 ? 1.0f / (float)a.pt_split : 0.0f;
@@ -178,10 +195,10 @@ hipError_t launch_mixed(int prec, const void *in, void *out, const MixedArgs &a,
 {
     const long long grid = (a.lines + a.tb - 1) / a.tb;
     const bool col = a.is != 1 || a.ois != 1;
-    const long long bytes = (prec == PREC_F64 ? 16LL : 8LL) * (col ? mixed_slots<true>(a.n, a.tb) : mixed_slots<false>(a.n, a.tb));
+    const long long bytes = (prec == PREC_F64 ? 16LL : 8LL) * (col ? mixed_slots<true>(a.n, a.tb, a.tbp) : mixed_slots<false>(a.n, a.tb, a.tbp));
     if (grid < 1 || grid > 0x7fffffffLL || a.nst < 1 || a.nst > MIXED_MAX_STAGES || a.tb < 1 ||
         (long long)a.tb * a.n > (long long)a.nt * a.cap || (a.nst > 1 && bytes > MIXED_LDS) ||
-        (a.nt > 512 && !col) || (a.pt_n && !col && a.nst > 1))
+        (a.nt > 512 && !col) || (col && a.nst > 1 && a.tbp < a.tb) || (a.pt_n && !col && a.nst > 1))
         return hipErrorInvalidValue;
     const unsigned g = (unsigned)grid;
     if (prec == PREC_F64)

@@ -7,7 +7,7 @@ namespace tope {
 template <typename R, int SIGN, int NT, bool COL, bool POST>
 static void launch(const void *in, void *out, const MixedArgs &a, unsigned grid, hipStream_t st)
 {
-    const size_t slots = (size_t)mixed_slots<COL>(a.n, a.tb);
+    const size_t slots = (size_t)mixed_slots<COL>(a.n, a.tb, a.tbp);
     hipLaunchKernelGGL((mixed_kernel<R, SIGN, NT, COL, POST>), dim3(grid), dim3(NT), slots * sizeof(cpx<R>), st,
                        static_cast<const cpx<R> *>(in), static_cast<cpx<R> *>(out), a);
 }

@@ -231,7 +231,8 @@ __device__ __forceinline__ void stage_at(int bi, const Stage &st, const Div32 &d
 }
 
 // LDS slot of element i of line t: lines back to back, or (COL) element by
-// element with the tile's lines side by side, an odd number of slots apart.
+// element with the tile's lines side by side, tbp slots from one element to
+// the next.
 // Both are linear in i, so the r slots of a butterfly are one base and a
 // uniform stride.  Reads are contiguous over the lanes and so are the writes
 // but a first stage's, r slots apart: mixed_plan puts a radix first that
@@ -242,16 +243,15 @@ __device__ __forceinline__ int slot_of(int t, int i, int n, int tbp)
     if constexpr (COL) return i * tbp + t;
     else return t * n + i;
 }
-__host__ __device__ __forceinline__ int mixed_tbp(int tb) { return tb | 1; }
 template <bool COL>
-__host__ __device__ __forceinline__ int mixed_slots(int n, int tb) { return COL ? n * mixed_tbp(tb) : n * tb; }
+__host__ __device__ __forceinline__ int mixed_slots(int n, int tb, int tbp) { return COL ? n * tbp : n * tb; }
 
 // LDS to registers and back.
 template <int r, typename R, int NT, bool COL>
 __device__ __forceinline__ void stage_get(cpx<R> (&v)[MIXED_E], const cpx<R> *lds, const Stage &st, int n, int tb,
-                                          const Div32 &dtb, int tid)
+                                          int tbp, const Div32 &dtb, int tid)
 {
-    const int tbp = mixed_tbp(tb), step = COL ? st.nb * tbp : st.nb;
+    const int step = COL ? st.nb * tbp : st.nb;
 #pragma unroll
     for (int b = 0; b < mixed_bf<r>(); ++b) {
         const int bi = tid + b * NT;
@@ -267,9 +267,9 @@ __device__ __forceinline__ void stage_get(cpx<R> (&v)[MIXED_E], const cpx<R> *ld
 
 template <int r, typename R, int NT, bool COL>
 __device__ __forceinline__ void stage_put(const cpx<R> (&v)[MIXED_E], cpx<R> *lds, const Stage &st, int n, int tb,
-                                          const Div32 &dtb, bool byline, int tid)
+                                          int tbp, const Div32 &dtb, bool byline, int tid)
 {
-    const int tbp = mixed_tbp(tb), step = COL ? st.Ns * tbp : st.Ns;
+    const int step = COL ? st.Ns * tbp : st.Ns;
 #pragma unroll
     for (int b = 0; b < mixed_bf<r>(); ++b) {
         const int bi = tid + b * NT;
@@ -470,7 +470,7 @@ mixed_kernel(const cpx<R> *in, cpx<R> *out, const MixedArgs a)
 {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     cpx<R> *lds = reinterpret_cast<cpx<R> *>(lds_raw);
-    const int n = a.n, tb = a.tb;
+    const int n = a.n, tb = a.tb, tbp = a.tbp;
     const Div32 dtb{tb, a.inv_tb};
     // strided lines share 128-byte segments with the neighbouring blocks'
     // lines: keep neighbours on one XCD (one L2)
@@ -494,7 +494,7 @@ mixed_kernel(const cpx<R> *in, cpx<R> *out, const MixedArgs a)
         const int tid = opaque_tid();                                           \
         stage_load<r, R, NT>(v, in, a, g, first, dtb, in_cols, tid);            \
         stage_run<r, SIGN, R, NT>(v, first, tb, tid);                           \
-        stage_put<r, R, NT, COL>(v, lds, first, n, tb, dtb, in_cols, tid);   \
+        stage_put<r, R, NT, COL>(v, lds, first, n, tb, tbp, dtb, in_cols, tid);   \
     }
     MIXED_SWITCH(first.r, MIXED_FIRST)
     for (int s = 1; s < a.nst - 1; ++s) {
@@ -506,10 +506,10 @@ mixed_kernel(const cpx<R> *in, cpx<R> *out, const MixedArgs a)
         cpx<R> w[mixed_bf<r>()][mixed_ntw<r>()]{};                              \
         stage_tw<r, R, NT, COL>(w, st, tb, dtb, tid);                           \
         __syncthreads();                                                        \
-        stage_get<r, R, NT, COL>(v, lds, st, n, tb, dtb, tid);                  \
+        stage_get<r, R, NT, COL>(v, lds, st, n, tb, tbp, dtb, tid);                  \
         __syncthreads();                                                        \
         stage_run_tw<r, SIGN, R, NT>(v, w, st, tb, tid);                        \
-        stage_put<r, R, NT, COL>(v, lds, st, n, tb, dtb, COL, tid);             \
+        stage_put<r, R, NT, COL>(v, lds, st, n, tb, tbp, dtb, COL, tid);             \
     }
         MIXED_SWITCH(st.r, MIXED_MID)
     }
@@ -522,7 +522,7 @@ mixed_kernel(const cpx<R> *in, cpx<R> *out, const MixedArgs a)
         cpx<R> w[mixed_bf<r>()][mixed_ntw<r>()]{};                              \
         stage_tw<r, R, NT, COL>(w, st, tb, dtb, tid);                           \
         __syncthreads();                                                        \
-        stage_get<r, R, NT, COL>(v, lds, st, n, tb, dtb, tid);                  \
+        stage_get<r, R, NT, COL>(v, lds, st, n, tb, tbp, dtb, tid);                  \
         stage_run_tw<r, SIGN, R, NT>(v, w, st, tb, tid);                        \
         stage_store<r, SIGN, R, NT, POST>(v, out, a, g, st, dtb, COL, tid);     \
     }
