@@ -130,6 +130,15 @@ struct MixedArgs {
     int pt_split;
     float inv_split;
 };
+// Half-spectrum step of the real-row pass: W_2n^k (k <= n), the distance of
+// the spectrum rows, DC and Nyquist packed in column 0, 1 / (points) of C2R.
+struct MixedReal {
+    const void *w;
+    long long pitch;
+    double scale;
+    int pack;
+    float inv_pairs;
+};
 bool mixed_supported(long long n);
 // 7-smooth n above MIXED_MAX_N that splits as n = n1 n2 with both factors
 // at most MIXED_MAX_N (mixed-radix four-step); *n1 >= n2 is the split used.
@@ -141,6 +150,11 @@ void mixed_schedule(MixedArgs &a, int prec);
 // a.twsize stage twiddles from the table W_n^i, i < n (forward sign)
 hipError_t gen_mixed_table(void *out, const void *roots, int prec, const MixedArgs &a, hipStream_t st);
 unsigned mixed_grid(const MixedArgs &a);
+// A real-row pass (rows of 2 a.n samples; in, out distinct arrays): R2C for
+// sign < 0, C2R for sign > 0.  mixed_real_supported: the lengths n it takes.
+bool mixed_real_supported(long long n);
+hipError_t launch_mixed_real(int prec, const void *in, void *out, const MixedArgs &a, MixedReal h, int sign,
+                             hipStream_t st);
 hipError_t launch_mixed(int prec, const void *in, void *out, const MixedArgs &a, int sign, hipStream_t st);
 struct ChirpGeo {
     long long O, os, C, cs, is;

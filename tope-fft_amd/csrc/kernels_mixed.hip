@@ -206,4 +206,25 @@ hipError_t launch_mixed(int prec, const void *in, void *out, const MixedArgs &a,
     return sign < 0 ? launch_mixed_t<float, -1>(in, out, a, g, st) : launch_mixed_t<float, 1>(in, out, a, g, st);
 }
 
+// n <= 16 (one thread a line) has no LDS tile to form the bins in.
+bool mixed_real_supported(long long n) { return n > 16 && mixed_supported(n); }
+
+hipError_t launch_mixed_real(int prec, const void *in, void *out, const MixedArgs &a, MixedReal h, int sign,
+                             hipStream_t st)
+{
+    const long long grid = (a.lines + a.tb - 1) / a.tb;
+    const long long bytes = (prec == PREC_F64 ? 16LL : 8LL) * a.n * a.tb;
+    if (grid < 1 || grid > 0x7fffffffLL || a.nst < 2 || a.nst > MIXED_MAX_STAGES || a.tb < 1 || a.is != 1 ||
+        a.ois != 1 || (a.nt != 256 && a.nt != 512) || (long long)a.tb * a.n > (long long)a.nt * a.cap ||
+        bytes > MIXED_LDS || a.pt_n || h.pitch <= a.n || in == out)
+        return hipErrorInvalidValue;
+    h.inv_pairs = 1.0f / (float)(a.n / 2 + 1);
+    const unsigned g = (unsigned)grid;
+    if (prec == PREC_F64)
+        return sign < 0 ? launch_mixed_real_t<double, -1>(in, out, a, h, g, st)
+                        : launch_mixed_real_t<double, 1>(in, out, a, h, g, st);
+    return sign < 0 ? launch_mixed_real_t<float, -1>(in, out, a, h, g, st)
+                    : launch_mixed_real_t<float, 1>(in, out, a, h, g, st);
+}
+
 }  // namespace tope

@@ -25,6 +25,7 @@
 // FZ = F0 + i Fm; after the inverse column passes column 0 holds
 // x0 + i xm, both real, and the row step reads X[0] = x0, X[m] = xm from it.
 #include "internal.hpp"
+#include "real_bins.hpp"
 
 namespace tope {
 
@@ -45,17 +46,8 @@ __global__ void r2c_post_kernel(const cpx<R> *__restrict__ Z, cpx<R> *__restrict
         x[0] = cpx<R>{zk.x + zk.y, zk.x - zk.y};
         return;
     }
-    // X[k] from a = Z[k], b = conj Z[m-k]; X[m-k] from a' = Z[m-k], b' = conj Z[k]
-    auto out = [&](cpx<R> a, cpx<R> bc, long long kk) {
-        const cpx<R> b{bc.x, -bc.y};
-        const cpx<R> e{R(0.5) * (a.x + b.x), R(0.5) * (a.y + b.y)};
-        // O = (a - b) / (2i) = (Im(a-b), -Re(a-b)) / 2
-        const cpx<R> o{R(0.5) * (a.y - b.y), R(-0.5) * (a.x - b.x)};
-        const cpx<R> wo = cmul(w[kk], o);
-        x[kk] = cpx<R>{e.x + wo.x, e.y + wo.y};
-    };
-    out(zk, zm, k);
-    if (m - k != k) out(zm, zk, m - k);
+    x[k] = r2c_bin(zk, zm, w[k]);
+    if (m - k != k) x[m - k] = r2c_bin(zm, zk, w[m - k]);
 }
 
 // Inverse: X (row pitch p) -> Z (row pitch m), scaled by s; one thread per pair.
@@ -74,16 +66,8 @@ __global__ void c2r_pre_kernel(const cpx<R> *__restrict__ X, cpx<R> *__restrict_
         xm = cpx<R>{xk.y, R(0)};
         xk = cpx<R>{xk.x, R(0)};
     }
-    auto out = [&](cpx<R> a, cpx<R> bc, long long kk) {
-        const cpx<R> b{bc.x, -bc.y};
-        const cpx<R> e{R(0.5) * (a.x + b.x), R(0.5) * (a.y + b.y)};
-        const cpx<R> d{R(0.5) * (a.x - b.x), R(0.5) * (a.y - b.y)};
-        const cpx<R> o = cmulc(d, w[kk]);  // d * conj(W^k)
-        // Z = E + i O
-        z[kk] = cpx<R>{s * (e.x - o.y), s * (e.y + o.x)};
-    };
-    if (k < m) out(xk, xm, k);
-    if (m - k != k && m - k < m) out(xm, xk, m - k);
+    z[k] = c2r_bin(xk, xm, w[k], s);  // k <= m / 2 < m
+    if (m - k != k && m - k < m) z[m - k] = c2r_bin(xm, xk, w[m - k], s);
 }
 
 // Fused rows: the m-point complex row transform and the half-spectrum step

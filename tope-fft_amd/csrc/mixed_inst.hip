@@ -41,6 +41,20 @@ hipError_t launch_mixed_t(const void *in, void *out, const MixedArgs &a, unsigne
     return hipGetLastError();
 }
 
+template <typename R, int SIGN>
+hipError_t launch_mixed_real_t(const void *in, void *out, const MixedArgs &a, const MixedReal &h, unsigned grid,
+                               hipStream_t st)
+{
+    const size_t bytes = (size_t)a.n * a.tb * sizeof(cpx<R>);
+    const cpx<R> *i = static_cast<const cpx<R> *>(in);
+    cpx<R> *o = static_cast<cpx<R> *>(out);
+    if (a.nt == 256) hipLaunchKernelGGL((mixed_real_kernel<R, SIGN, 256>), dim3(grid), dim3(256), bytes, st, i, o, a, h);
+    else hipLaunchKernelGGL((mixed_real_kernel<R, SIGN, 512>), dim3(grid), dim3(512), bytes, st, i, o, a, h);
+    return hipGetLastError();
+}
+
 template hipError_t launch_mixed_t<MIXED_R, MIXED_SIGN>(const void *, void *, const MixedArgs &, unsigned, hipStream_t);
+template hipError_t launch_mixed_real_t<MIXED_R, MIXED_SIGN>(const void *, void *, const MixedArgs &, const MixedReal &,
+                                                             unsigned, hipStream_t);
 
 }  // namespace tope
