@@ -125,7 +125,7 @@ struct Pass {
     long long dft_n = 0;
     const void *dft_roots = nullptr;
     const void *real_w = nullptr;  // PASS_REAL: W_n^k, k = 0..m (FP64)
-    const void *real_stw = nullptr;  // PASS_REAL fused with the row transform: stage table of (m, 16)
+    const void *real_stw = nullptr;  // PASS_REAL fused with the row transform: stage table of (m, real_rows_elems(m))
     bool real_mixed = false;         // PASS_REAL fused with mixed-radix rows (mx)
     int fixed_dir = -1;            // >= 0: the pass always runs in this direction (Bluestein's inner FFTs)
     int chirp_op = 0;              // PASS_CHIRP: CHIRP_PRE / CHIRP_MUL / CHIRP_POST
@@ -1656,12 +1656,12 @@ int build_real_plan(struct topeFFT *f, long long nx, long long ny, long long nz,
         ps.name = "real_half_spectrum";
         if (fused) {
             void *stw = nullptr;
-            err = pl.stage_table((int)m, 16, &stw);
+            err = pl.stage_table((int)m, real_rows_elems(m), &stw);
             if (err != hipSuccess) return fail(map_err(err));
             ps.real_stw = stw;
             ps.name = "real_rows_fused";
             P->axis_tw[0].n = (int)m;
-            P->axis_tw[0].e = 16;
+            P->axis_tw[0].e = real_rows_elems(m);
             P->axis_tw[0].table = stw;
         }
         if (fused_mixed) {

@@ -83,8 +83,10 @@ hipError_t launch_real_pass(int prec, int dir, const void *in, void *out, const 
 // The m-point row transform fused with that step (64 <= m <= 4096, powers of
 // two): dir 0 reads the real rows (pitch m complex) and writes the half
 // spectrum, dir 1 the reverse (scaled by s); stw is the stage twiddle table
-// of schedule (m, 16).
+// of schedule (m, real_rows_elems(m)).
 bool real_rows_supported(long long m);
+// Elements a thread holds in a fused row of m points.
+constexpr int real_rows_elems(long long m) { return m < 4096 ? 8 : 16; }
 hipError_t launch_real_rows(int prec, int dir, const void *in, void *out, const void *stw, const void *w, long long m,
                             long long pitch, long long rows, double s, int pack, hipStream_t st);
 // Packed DC/Nyquist columns of the half spectrum X (rows K = ky + ny kz at

@@ -79,6 +79,13 @@ __global__ void c2r_pre_kernel(const cpx<R> *__restrict__ X, cpx<R> *__restrict_
 //   0), store the row of m + 1 values at `pitch`.
 //   C2R (SIGN = +1): load X[k] and X[m - k] for its k, form
 //   Z[k] = s (E[k] + i O[k]), run the inverse radix stages, store z.
+// What bounds it: memory for many rows, the latency of the stages for few.
+// Eight elements a thread (64 or 128 threads a block, 256 at 2048 points) put
+// twice the waves of sixteen on a row: R2C and C2R of 4096 x 4096 complex128
+// 248 -> 244 us, 2048 x 4096 141 -> 136, 1024 x 512 27.1 -> 21.8, 128 x 128
+// 16.1 -> 13.7, complex64 1024 x 512 28.5 -> 24.0.  4096 points keep sixteen:
+// 8192 x 2048 226 us, 228 with eight (complex64 129.9 and 129.1).  Four:
+// 1024 x 4096 97.6 us against 95.1, complex64 2048 x 4096 89.2 against 84.1.
 template <typename R, int N, int E, int TB, int SIGN>
 __global__ void __launch_bounds__(TB *(N / E))
 real_rows_kernel(const cpx<R> *__restrict__ in, cpx<R> *__restrict__ out,
@@ -192,13 +199,13 @@ static hipError_t launch_real_rows_t(int dir, const void *in, void *out, const v
                                      long long pitch, long long rows, double s, int pack, hipStream_t st)
 {
     switch (m) {
-    case 64: return launch_rows_t<R, 64, 16, 16>(dir, in, out, stw, w, pitch, rows, s, pack, st);
-    case 128: return launch_rows_t<R, 128, 16, 16>(dir, in, out, stw, w, pitch, rows, s, pack, st);
-    case 256: return launch_rows_t<R, 256, 16, 16>(dir, in, out, stw, w, pitch, rows, s, pack, st);
-    case 512: return launch_rows_t<R, 512, 16, 8>(dir, in, out, stw, w, pitch, rows, s, pack, st);
-    case 1024: return launch_rows_t<R, 1024, 16, 4>(dir, in, out, stw, w, pitch, rows, s, pack, st);
-    case 2048: return launch_rows_t<R, 2048, 16, 2>(dir, in, out, stw, w, pitch, rows, s, pack, st);
-    case 4096: return launch_rows_t<R, 4096, 16, 1>(dir, in, out, stw, w, pitch, rows, s, pack, st);
+    case 64: return launch_rows_t<R, 64, real_rows_elems(64), 8>(dir, in, out, stw, w, pitch, rows, s, pack, st);
+    case 128: return launch_rows_t<R, 128, real_rows_elems(128), 8>(dir, in, out, stw, w, pitch, rows, s, pack, st);
+    case 256: return launch_rows_t<R, 256, real_rows_elems(256), 4>(dir, in, out, stw, w, pitch, rows, s, pack, st);
+    case 512: return launch_rows_t<R, 512, real_rows_elems(512), 2>(dir, in, out, stw, w, pitch, rows, s, pack, st);
+    case 1024: return launch_rows_t<R, 1024, real_rows_elems(1024), 1>(dir, in, out, stw, w, pitch, rows, s, pack, st);
+    case 2048: return launch_rows_t<R, 2048, real_rows_elems(2048), 1>(dir, in, out, stw, w, pitch, rows, s, pack, st);
+    case 4096: return launch_rows_t<R, 4096, real_rows_elems(4096), 1>(dir, in, out, stw, w, pitch, rows, s, pack, st);
     default: return hipErrorInvalidValue;
     }
 }
