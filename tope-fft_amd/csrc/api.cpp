@@ -101,6 +101,7 @@ enum PassKind {
     PASS_CHIRP = 5,
     PASS_MIXED = 6,
     PASS_CHIRP_LINE = 8,  // Bluestein lines inside a workgroup
+    PASS_CHIRP_ROWS = 10,  // contiguous Bluestein lines in three passes
     PASS_DONE = 9,        // a step that the launch before it has carried out
     PASS_RPACK = 7  // real plans: unpack (FORWARD) / pack (INVERSE) of the DC/Nyquist columns
 };
@@ -133,6 +134,7 @@ struct Pass {
     ChirpGeo chirp_g{1, 0, 1, 0, 1};
     const void *chirp_tab[2] = {nullptr, nullptr};  // transformed filters, forward / inverse
     ChirpLineArgs cl{};                             // PASS_CHIRP_LINE
+    ChirpRowsArgs cr{};                             // PASS_CHIRP_ROWS, chirp_op
     MixedArgs mx{};                                 // PASS_MIXED
     const char *name = "";
 };
@@ -702,8 +704,9 @@ class Planner {
 
     // Non-power-of-two axis of length n (lines g) by Bluestein's identity
     // (kernels_chirp.hip).  M <= CHIRP_MAX_M: one in-place pass, each line's
-    // convolution inside a workgroup (bluestein_lines).  Longer: chirp pre-multiply of every line into its own
-    // zero-padded row of M elements in the other buffer, forward FFT_M over
+    // convolution inside a workgroup (bluestein_lines).  Contiguous lines up
+    // to M = CHIRP_ROWS_M: three passes through padded rows in the other
+    // buffer.  Else: chirp pre-multiply of every line into its own zero-padded row of M elements in the other buffer, forward FFT_M over
     // the rows, product with the transformed filter of the direction,
     // inverse FFT_M (both inner FFTs keep their direction whatever the outer
     // one), chirp post-multiply back into the line.  The data stays in
@@ -865,10 +868,38 @@ class Planner {
         return TOPE_SUCCESS;
     }
 
+    // Tables of the three-pass form of contiguous lines (filter apart).
+    int chirp_rows_args(long long n, long long M, const Geo &g, ChirpRowsArgs *a)
+    {
+        int lg = 0;
+        while ((1LL << lg) < M) ++lg;
+        a->g = ChirpGeo{g.O, g.os, g.C, g.cs, g.is};
+        a->n = (int)n;
+        a->M = (int)M;
+        a->n1 = 1 << lg / 2;
+        a->n2 = (int)(M >> lg / 2);
+        a->shift = (lg + 1) / 2;
+        void *tw1 = nullptr, *tw2 = nullptr, *lo = nullptr, *hi = nullptr, *ct = nullptr;
+        hipError_t err = stage_table(a->n1, 8, &tw1);
+        if (err == hipSuccess) err = stage_table(a->n2, 8, &tw2);
+        if (err == hipSuccess) err = power_table(M, 1, 1LL << a->shift, &lo);
+        if (err == hipSuccess) err = power_table(M, 1LL << a->shift, M >> a->shift, &hi);
+        if (err == hipSuccess) err = hipMalloc(&ct, (size_t)n * 16);
+        if (err != hipSuccess) return map_err(err);
+        P->allocs.push_back(ct);
+        a->tw1 = tw1;
+        a->tw2 = tw2;
+        a->lo = lo;
+        a->hi = hi;
+        a->chirp = ct;
+        return map_err(gen_chirp_table(ct, n, st));
+    }
+
     int bluestein_axis(long long n, const Geo &g, int *cur)
     {
         const long long M = chirp_len(n), lines = g.O * g.C;
         if (chirp_fused(M)) return bluestein_lines(n, M, g, *cur);
+        const bool rows3 = g.is == 1 && M <= CHIRP_ROWS_M;
         const int data = *cur, scratch = *cur ^ 1;
         const size_t tb = (size_t)M * 16;
         void *tab[2] = {nullptr, nullptr};
@@ -891,6 +922,20 @@ class Planner {
             ps.name = op == CHIRP_PRE ? "chirp_pre" : op == CHIRP_MUL ? "chirp_mul" : "chirp_post";
             P->passes.push_back(ps);
         };
+        if (rows3) {
+            ChirpRowsArgs ra{};
+            int rc3 = chirp_rows_args(n, M, g, &ra);
+            if (rc3) return rc3;
+            auto rows_pass = [&](int op, int bi, int bo) {
+                chirp_pass(op, bi, bo);
+                P->passes.back().kind = PASS_CHIRP_ROWS;
+                P->passes.back().cr = ra;
+            };
+            rows_pass(CHIRP_PRE, data, scratch);
+            rows_pass(CHIRP_MUL, scratch, scratch);
+            rows_pass(CHIRP_POST, scratch, data);
+            return chirp_filters(n, M, scratch, tab, ra.n1, ra.n2);
+        }
         // the rows live in the scratch buffer; an inner FFT longer than one
         // pass uses the data buffer as its intermediate: the pre-multiply
         // has read every line of the axis (the whole array) by then
@@ -907,11 +952,17 @@ class Planner {
         for (size_t i = f1; i < P->passes.size(); ++i) P->passes[i].fixed_dir = INVERSE;
         chirp_pass(CHIRP_POST, rc_, data);
 
-        // transformed filters: b into the scratch buffer, a one-row forward
-        // FFT_M (planned, run, then dropped from the pass list), copy out
+        return chirp_filters(n, M, scratch, tab, 0, 0);
+    }
+
+    // Transformed filters: b into the scratch buffer, a one-row forward FFT_M
+    // (planned, run, then dropped from the pass list), copy out, for n1 > 0 in
+    // the order of the three-pass form.
+    int chirp_filters(long long n, long long M, int scratch, void *const tab[2], int n1, int n2)
+    {
         const size_t g0 = P->passes.size();
         int fc = scratch;
-        rc = axis(M, Geo{1, 0, 1, M, 1}, &fc, -1);
+        int rc = axis(M, Geo{1, 0, 1, M, 1}, &fc, -1);
         if (rc) return rc;
         const size_t g1 = P->passes.size();
         for (int d = 0; d < 2 && !rc; ++d) {
@@ -919,7 +970,9 @@ class Planner {
                 launch_chirp(CHIRP_FILTER, nullptr, P->buf[scratch], nullptr, ChirpGeo{1, 0, 1, 0, 1}, n, M, 1.0, d, st);
             for (size_t i = g0; i < g1 && err == hipSuccess; ++i)
                 if (launch_pass(P, i, st, FORWARD)) err = hipErrorUnknown;
-            if (err == hipSuccess) err = hipMemcpyAsync(tab[d], P->buf[fc], tb, hipMemcpyDeviceToDevice, st);
+            if (err == hipSuccess)
+                err = n1 ? gen_chirp_order(P->buf[fc], tab[d], n1, n2, st)
+                         : hipMemcpyAsync(tab[d], P->buf[fc], (size_t)M * 16, hipMemcpyDeviceToDevice, st);
             if (err != hipSuccess) rc = map_err(err);
         }
         P->passes.resize(g0);
@@ -1157,6 +1210,13 @@ int launch_pass(PlanImpl *P, size_t i, hipStream_t s, int dir, long long rep0, l
         c.filter = ps.chirp_tab[c.inverse];
         c.scale = (1.0 / (double)c.M) * (ps.last ? sc : 1.0);
         hipError_t err = launch_chirp_lines(ib, ob, c, s);
+        if (err != hipSuccess) return map_err(err);
+    } else if (ps.kind == PASS_CHIRP_ROWS) {
+        ChirpRowsArgs c = ps.cr;
+        c.inverse = dir == INVERSE ? 1 : 0;
+        c.filter = ps.chirp_tab[c.inverse];
+        c.scale = (1.0 / (double)c.M) * (ps.last ? sc : 1.0);
+        hipError_t err = launch_chirp_rows(ps.chirp_op, ib, ob, c, s);
         if (err != hipSuccess) return map_err(err);
     } else if (ps.kind == PASS_CHIRP) {
         // 1/M undoes the unnormalised inner inverse FFT; the plan's 1/N of

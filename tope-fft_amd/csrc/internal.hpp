@@ -172,6 +172,19 @@ struct ChirpLineArgs {
     const void *chirp, *filter, *tw;
     double scale;  // 1/M, times the plan's 1/N on the last inverse pass
 };
+// Contiguous lines (g.is = 1) with CHIRP_MAX_M < M <= CHIRP_ROWS_M in three
+// passes over rows of M elements: M = n1 n2, tw1 / tw2 the stage tables of
+// (n1, 8) and (n2, 8), W_M^x = lo[x mod 2^shift] hi[x >> shift], filter in the
+// order that gen_chirp_order leaves.
+constexpr long long CHIRP_ROWS_M = 1LL << 24;
+struct ChirpRowsArgs {
+    ChirpGeo g;
+    int n, M, n1, n2, inverse, shift;
+    const void *chirp, *filter, *tw1, *tw2, *lo, *hi;
+    double scale;
+};
+hipError_t launch_chirp_rows(int op, const void *in, void *out, const ChirpRowsArgs &a, hipStream_t st);
+hipError_t gen_chirp_order(const void *in, void *out, int n1, int n2, hipStream_t st);
 hipError_t gen_chirp_table(void *out, long long n, hipStream_t st);
 hipError_t launch_chirp_lines(const void *in, void *out, const ChirpLineArgs &a, hipStream_t st);
 hipError_t launch_chirp(int op, const void *in, void *out, const void *table, const ChirpGeo &g, long long n,

@@ -12,7 +12,8 @@
 // The inverse transform uses conj(c) throughout.  Every line of an axis is
 // padded into its own row of M elements of a scratch array, so the two inner
 // FFTs are contiguous row passes.  Up to M = CHIRP_MAX_M a line's whole
-// convolution runs in one workgroup instead (chirp_line_kernel).
+// convolution runs in one workgroup instead (chirp_line_kernel), contiguous
+// lines up to M = CHIRP_ROWS_M take three passes (chirp_cols_kernel).
 #include "internal.hpp"
 
 namespace tope {
@@ -124,6 +125,123 @@ chirp_line_kernel(const cpx<double> *in, cpx<double> *out, const ChirpLineArgs a
     }
 }
 
+// Longer contiguous lines, M = n1 n2, element i = i1 n2 + i2 of a row of the
+// padded array, bin k = k1 + n1 k2.  The forward transform's second half and the
+// inverse's first half work on the same n2 contiguous elements (one k1), so a
+// line's convolution is three passes and the bins are never put in order:
+//   chirp_cols_kernel<PRE>   chirp, transforms over i1, W_M^(i2 k1)
+//   chirp_mid_kernel         transform over i2, filter (kept in this order),
+//                            inverse transform over k2
+//   chirp_cols_kernel<POST>  W_M^-(i2 k1), inverse over k1, chirp, 1/M
+// What bounds it: launches and latency at one line, else the memory of the
+// padded rows, written twice and read twice (seven passes wrote them six
+// times, with a sincospi for every element at both ends).
+// A forward and an inverse transform: 3001 points 55 -> 23 us, 20011 55 -> 26,
+// 300007 135 -> 68, 1000003 210 -> 116, 100 lines of 32771 954 -> 410.  Eight
+// elements a thread; sixteen take 28, 29, 70, 111 and 467 us.
+constexpr int CR_E = 8;
+// v[e] *= W_M^(b (p + P e)) (SIGN < 0) or its conjugate: four table values
+// and at most three products to a factor.
+template <int SIGN>
+__device__ __forceinline__ void chirp_twiddle(cpx<double> (&v)[CR_E], int b, int p, int P, const ChirpRowsArgs &a)
+{
+    const cpx<double> *lo = static_cast<const cpx<double> *>(a.lo), *hi = static_cast<const cpx<double> *>(a.hi);
+    auto at = [&](int k) { return pt_lookup((long long)b * k, lo, hi, (long long)a.M, a.shift); };
+    const cpx<double> s1 = at(P), s2 = at(2 * P), s4 = at(4 * P);
+    cpx<double> w[4];
+    w[0] = at(p);
+    w[1] = cmul(w[0], s1);
+    w[2] = cmul(w[0], s2);
+    w[3] = cmul(w[1], s2);
+#pragma unroll
+    for (int e = 0; e < CR_E; ++e) v[e] = twmul<SIGN>(v[e], e < 4 ? w[e & 3] : cmul(w[e & 3], s4));
+}
+
+template <int N, int TB, bool POST>
+__global__ void __launch_bounds__(TB *(N / CR_E))
+chirp_cols_kernel(const cpx<double> *in, cpx<double> *out, const ChirpRowsArgs a)
+{
+    using R = double;
+    constexpr int E = CR_E, P = N / E, H = E / 2;  // n <= M / 2: e >= H is padding
+    __shared__ __align__(16) unsigned char lds[Exchange<R, N, E, TB, true, true>::BYTES];
+    const int tid = threadIdx.x, t = tid % TB, p = tid / TB;
+    const cpx<R> *tw = static_cast<const cpx<R> *>(a.tw1);
+    const cpx<R> *ct = static_cast<const cpx<R> *>(a.chirp);
+
+    const long long blk = xcd_block(1);
+    const int tiles = a.n2 / TB;
+    const long long l = blk / tiles;
+    const int i2 = (int)(blk - l * tiles) * TB + t;
+    const long long o = l / a.g.C, c = l - o * a.g.C;
+    const long long at = o * a.g.os + c * a.g.cs, row = l * a.M;
+
+    cpx<R> v[E];
+    if constexpr (!POST) {
+#pragma unroll
+        for (int e = 0; e < H; ++e) {
+            const int i = (p + P * e) * a.n2 + i2;
+            v[e] = i < a.n ? in[at + i] : cpx<R>{0, 0};
+        }
+#pragma unroll
+        for (int e = 0; e < H; ++e) {
+            const int i = (p + P * e) * a.n2 + i2;
+            const cpx<R> w = ct[i < a.n ? i : 0];
+            v[e] = a.inverse ? cmulc(v[e], w) : cmul(v[e], w);
+        }
+#pragma unroll
+        for (int e = H; e < E; ++e) v[e] = cpx<R>{0, 0};
+        run_stages<R, N, E, TB, true, true, -1, 0>(v, p, t, tw, lds);
+        chirp_twiddle<-1>(v, i2, p, P, a);
+#pragma unroll
+        for (int e = 0; e < E; ++e) out[row + (p + P * e) * a.n2 + i2] = v[e];
+    } else {
+#pragma unroll
+        for (int e = 0; e < E; ++e) v[e] = in[row + (p + P * e) * a.n2 + i2];
+        chirp_twiddle<1>(v, i2, p, P, a);
+        run_stages<R, N, E, TB, true, true, 1, 0>(v, p, t, tw, lds);
+#pragma unroll
+        for (int e = 0; e < H; ++e) {
+            const int i = (p + P * e) * a.n2 + i2;
+            if (i < a.n) {
+                const cpx<R> w = ct[i];
+                const cpx<R> r = a.inverse ? cmulc(v[e], w) : cmul(v[e], w);
+                out[at + i] = cpx<R>{r.x * a.scale, r.y * a.scale};
+            }
+        }
+    }
+}
+
+template <int N, int TB>
+__global__ void __launch_bounds__(TB *(N / CR_E)) chirp_mid_kernel(cpx<double> *S, const ChirpRowsArgs a)
+{
+    using R = double;
+    constexpr int E = CR_E, P = N / E;
+    __shared__ __align__(16) unsigned char lds[Exchange<R, N, E, TB, false, true>::BYTES];
+    const int tid = threadIdx.x, t = tid / P, p = tid % P;
+    const cpx<R> *tw = static_cast<const cpx<R> *>(a.tw2);
+    const long long row = xcd_block(0) * TB + t;
+    cpx<R> *s = S + row * N;
+    const cpx<R> *fl = static_cast<const cpx<R> *>(a.filter) + (row & (a.n1 - 1)) * N;
+
+    cpx<R> v[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) v[e] = s[p + P * e];
+    run_stages<R, N, E, TB, false, true, -1, 0>(v, p, t, tw, lds);
+#pragma unroll
+    for (int e = 0; e < E; ++e) v[e] = cmul(v[e], fl[p + P * e]);
+    __syncthreads();  // the forward transform's last exchange has been read
+    run_stages<R, N, E, TB, false, true, 1, 0>(v, p, t, tw, lds);
+#pragma unroll
+    for (int e = 0; e < E; ++e) s[p + P * e] = v[e];
+}
+
+// out[k1 n2 + k2] = in[k1 + n1 k2]
+__global__ void chirp_order_kernel(const cpx<double> *in, cpx<double> *out, int n1, int n2)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n1 * n2) out[i] = in[i / n2 + n1 * (i % n2)];
+}
+
 // Element k of line l (o = l / C, c = l % C) of the axis: o os + c cs + k is.
 // Threads run along k when the axis is contiguous (is = 1), else along the
 // lines (adjacent lines are adjacent in memory for the strided axes).
@@ -213,6 +331,64 @@ hipError_t launch_chirp_lines(const void *in, void *out, const ChirpLineArgs &a,
     case 4096: return launch_line_n<4096, 1, 4, 2>(in, out, a, st);
     default: return hipErrorInvalidValue;
     }
+}
+
+template <int N, int TB>
+static hipError_t launch_cols_t(int op, const void *in, void *out, const ChirpRowsArgs &a, hipStream_t st)
+{
+    const long long grid = a.g.O * a.g.C * (a.n2 / TB);
+    if (grid < 1 || grid > 0x7fffffffLL || a.n2 % TB) return hipErrorInvalidValue;
+    const cpx<double> *i = static_cast<const cpx<double> *>(in);
+    cpx<double> *o = static_cast<cpx<double> *>(out);
+    if (op == CHIRP_PRE)
+        hipLaunchKernelGGL((chirp_cols_kernel<N, TB, false>), dim3((unsigned)grid), dim3(TB * (N / CR_E)), 0, st, i, o, a);
+    else
+        hipLaunchKernelGGL((chirp_cols_kernel<N, TB, true>), dim3((unsigned)grid), dim3(TB * (N / CR_E)), 0, st, i, o, a);
+    return hipGetLastError();
+}
+
+template <int N, int TB>
+static hipError_t launch_mid_t(void *S, const ChirpRowsArgs &a, hipStream_t st)
+{
+    const long long rows = a.g.O * a.g.C * a.n1, grid = rows / TB;
+    if (grid < 1 || grid > 0x7fffffffLL || rows % TB) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((chirp_mid_kernel<N, TB>), dim3((unsigned)grid), dim3(TB * (N / CR_E)), 0, st,
+                       static_cast<cpx<double> *>(S), a);
+    return hipGetLastError();
+}
+
+hipError_t launch_chirp_rows(int op, const void *in, void *out, const ChirpRowsArgs &a, hipStream_t st)
+{
+    if (a.n < 1 || 2LL * a.n - 1 > a.M || a.g.is != 1 || (long long)a.n1 * a.n2 != a.M || a.M > CHIRP_ROWS_M)
+        return hipErrorInvalidValue;
+    if (op == CHIRP_MUL) {
+        switch (a.n2) {  // 64 threads or one row a block
+        case 128: return launch_mid_t<128, 4>(out, a, st);
+        case 256: return launch_mid_t<256, 2>(out, a, st);
+        case 512: return launch_mid_t<512, 1>(out, a, st);
+        case 1024: return launch_mid_t<1024, 1>(out, a, st);
+        case 2048: return launch_mid_t<2048, 1>(out, a, st);
+        case 4096: return launch_mid_t<4096, 1>(out, a, st);
+        default: return hipErrorInvalidValue;
+        }
+    }
+    switch (a.n1) {  // 64- to 128-byte row segments while 1024 threads hold them
+    case 64: return launch_cols_t<64, 8>(op, in, out, a, st);
+    case 128: return launch_cols_t<128, 4>(op, in, out, a, st);
+    case 256: return launch_cols_t<256, 4>(op, in, out, a, st);
+    case 512: return launch_cols_t<512, 4>(op, in, out, a, st);
+    case 1024: return launch_cols_t<1024, 4>(op, in, out, a, st);
+    case 2048: return launch_cols_t<2048, 4>(op, in, out, a, st);
+    case 4096: return launch_cols_t<4096, 2>(op, in, out, a, st);
+    default: return hipErrorInvalidValue;
+    }
+}
+
+hipError_t gen_chirp_order(const void *in, void *out, int n1, int n2, hipStream_t st)
+{
+    hipLaunchKernelGGL(chirp_order_kernel, dim3((unsigned)((n1 * n2 + 255) / 256)), dim3(256), 0, st,
+                       static_cast<const cpx<double> *>(in), static_cast<cpx<double> *>(out), n1, n2);
+    return hipGetLastError();
 }
 
 hipError_t gen_chirp_table(void *out, long long n, hipStream_t st)
