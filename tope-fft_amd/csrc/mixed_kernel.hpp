@@ -23,7 +23,7 @@
 // blocks on a CU.
 // A forward and an inverse transform, against radices 2, 3, 4, 5, 7, 8, 16
 // between two LDS buffers with roots from a two-level table: 3000^2 648 ->
-// 329 us (rows 160 -> 74 us, 3.9 TB/s; columns 172 -> 92 us: a tile of three
+// 323 us (rows 160 -> 74 us, 3.9 TB/s; columns 172 -> 92 us: a tile of three
 // lines fills the LDS, so one block per CU alternates between memory and
 // arithmetic), 100^3 85 -> 63.5 us, 1000^2 52 us, complex64 100^3 45 us.
 // Twiddles read ahead of the barrier before their stage: 1-3 % of that.
