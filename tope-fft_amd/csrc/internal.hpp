@@ -114,7 +114,7 @@ struct MixedArgs {
     long long O, os, C, cs, is, lines;
     int n, nst;
     MixedStage st[MIXED_MAX_STAGES];
-    int cap;         // elements a thread can hold at the list's radices
+    int e, cap;      // elements a thread holds, and can hold at the list's radices
     int twsize;      // entries of the stage table
     int nt, tb;      // threads and lines per block
     int tbp;         // LDS slots between the elements of a strided line

@@ -43,7 +43,7 @@ bool mixed_supported(long long n)
 }
 
 // Elements a thread can hold at radix r.
-static int mixed_cap(int r) { return MIXED_E / r * r; }
+static int mixed_cap(int r, int e = MIXED_E) { return e / r * r; }
 
 // Fewest radices of 2 .. 16 whose product is n; of those lists the one whose
 // smallest mixed_cap is largest (more elements a thread), then the most
@@ -98,7 +98,7 @@ void mixed_schedule(MixedArgs &a, int prec)
 {
     std::vector<int> rad = mixed_radices(a.n);
     a.nst = (int)rad.size();
-    a.cap = MIXED_E;
+    a.e = a.cap = MIXED_E;
     for (int r : rad) a.cap = std::min(a.cap, mixed_cap(r));
 
     // Tile: 256 threads, or as many more as a line (rows) or a 64-byte wide
@@ -110,20 +110,19 @@ void mixed_schedule(MixedArgs &a, int prec)
     // 48 x 60 x 56 40.0 -> 33.3 us (a forward and an inverse transform).
     // Strided lines take rows in segments of tb elements, and below 64 bytes
     // each costs more than its bytes: 2400 x 2400 takes 182 us in segments of
-    // 64 bytes, 208 to 210 in 32 or 48 and 281 in 16 (its rows 88 of each).  A
+    // 64 bytes, 208 to 210 in 32 or 48 and 281 in 16 (its rows 88 of each);
+    // complex64 115 in 32, 132 in 24, 137 in 16.  A
     // higher factor for 32 bytes loses where those tiles fill the chip better:
     // 900 x 900 50.7 us in 32 bytes, 55.5 in 16.
     const int eb = prec == PREC_F64 ? 16 : 8;
     const bool col = a.is != 1 || a.ois != 1;
     const int want = col ? 64 / eb : 1;
-    a.nt = 256;
     a.tbp = 1;
-    if (a.nst == 1) {
-        a.tb = 256;
-    } else {
-        while (a.nt < (col ? 1024 : 512) && a.nt * a.cap < want * a.n) a.nt *= 2;
-        const int most = std::max(1, std::min(a.nt * a.cap / a.n, 64));
-        double best = 0;
+    double best = 0;
+    // the line count of least cost for threads of e elements
+    auto tile = [&](int e, int cap, int nt, int most) {
+        while (nt < (col ? 1024 : 512) && nt * cap < want * a.n) nt *= 2;
+        most = std::max(1, std::min(nt * cap / a.n, most));
         for (int tb = most; tb >= 1; --tb) {
             if (tb != most && tb > want && tb % want) continue;  // whole 64-byte segments
             // an odd distance between a line's elements spreads the first
@@ -133,12 +132,30 @@ void mixed_schedule(MixedArgs &a, int prec)
             if (col && (long long)a.n * tbp * eb > MIXED_LDS) tbp = tb;
             const long long bytes = (long long)eb * (col ? mixed_slots<true>(a.n, tb, tbp) : mixed_slots<false>(a.n, tb, tbp));
             if (bytes > MIXED_LDS) continue;
-            const long long slots = 256 * std::min<long long>(MIXED_LDS / bytes, 1024 / a.nt);
+            const long long slots = 256 * std::min<long long>(MIXED_LDS / bytes, 1024 / nt);
             const long long blocks = (a.lines + tb - 1) / tb;
             const int seg = col ? tb * eb : 64;  // bytes of a row that a tile takes
-            const double mem = seg < 32 ? 1.9 : seg < 64 ? 1.2 : 1.0;
+            const double mem = seg < 24 ? 1.9 : seg < 32 ? 1.45 : seg < 64 ? 1.2 : 1.0;
             const double cost = (double)((blocks + slots - 1) / slots) * ((double)tb * a.n + 1000.0) * mem;
-            if (best == 0 || cost < best) best = cost, a.tb = tb, a.tbp = tbp;
+            if (best == 0 || cost < best) best = cost, a.tb = tb, a.tbp = tbp, a.nt = nt, a.e = e, a.cap = cap;
+        }
+    };
+    if (a.nst == 1) {
+        a.nt = 256;
+        a.tb = 256;
+    } else {
+        tile(MIXED_E, a.cap, 256, 64);
+        // complex64 columns of which 1024 threads hold fewer than four at 16
+        // elements each (lengths above 2400 with radices that waste some):
+        // 32 elements, three or four lines, where they cost less.  4000 x 4000
+        // 354 -> 308 us, 1080 x 4000 155 -> 121, 600 x 3645 99 -> 72 (forward
+        // and inverse); not 1050 x 2430, three lines of 16 elements a thread
+        // 84, four of 32 95, nor 500 x 4000, 67 and 68.  Five and more lines, whose segments
+        // straddle 32 bytes, lose: 3600^2 219 -> 247.
+        if (prec == PREC_F32 && col && 4 * a.n > 1024 * a.cap) {
+            int cap = MIXED_WIDE;
+            for (int r : rad) cap = std::min(cap, mixed_cap(r, MIXED_WIDE));
+            tile(MIXED_WIDE, cap, 1024, 4);
         }
     }
     if (a.tb > a.lines) {
@@ -198,7 +215,8 @@ hipError_t launch_mixed(int prec, const void *in, void *out, const MixedArgs &a,
     const long long bytes = (prec == PREC_F64 ? 16LL : 8LL) * (col ? mixed_slots<true>(a.n, a.tb, a.tbp) : mixed_slots<false>(a.n, a.tb, a.tbp));
     if (grid < 1 || grid > 0x7fffffffLL || a.nst < 1 || a.nst > MIXED_MAX_STAGES || a.tb < 1 ||
         (long long)a.tb * a.n > (long long)a.nt * a.cap || (a.nst > 1 && bytes > MIXED_LDS) ||
-        (a.nt > 512 && !col) || (col && a.nst > 1 && a.tbp < a.tb) || (a.pt_n && !col && a.nst > 1))
+        (a.nt > 512 && !col) || (a.e != MIXED_E && (a.nt != 1024 || !col || prec != PREC_F32)) ||
+        (col && a.nst > 1 && a.tbp < a.tb) || (a.pt_n && !col && a.nst > 1))
         return hipErrorInvalidValue;
     const unsigned g = (unsigned)grid;
     if (prec == PREC_F64)
@@ -214,7 +232,7 @@ hipError_t launch_mixed_real(int prec, const void *in, void *out, const MixedArg
 {
     const long long grid = (a.lines + a.tb - 1) / a.tb;
     const long long bytes = (prec == PREC_F64 ? 16LL : 8LL) * a.n * a.tb;
-    if (grid < 1 || grid > 0x7fffffffLL || a.nst < 2 || a.nst > MIXED_MAX_STAGES || a.tb < 1 || a.is != 1 ||
+    if (grid < 1 || grid > 0x7fffffffLL || a.nst < 2 || a.nst > MIXED_MAX_STAGES || a.e != MIXED_E || a.tb < 1 || a.is != 1 ||
         a.ois != 1 || (a.nt != 256 && a.nt != 512) || (long long)a.tb * a.n > (long long)a.nt * a.cap ||
         bytes > MIXED_LDS || a.pt_n || h.pitch <= a.n || in == out)
         return hipErrorInvalidValue;

@@ -4,17 +4,23 @@
 
 namespace tope {
 
-template <typename R, int SIGN, int NT, bool COL, bool POST>
+template <typename R, int SIGN, int NT, bool COL, bool POST, int E = MIXED_E>
 static void launch(const void *in, void *out, const MixedArgs &a, unsigned grid, hipStream_t st)
 {
     const size_t slots = (size_t)mixed_slots<COL>(a.n, a.tb, a.tbp);
-    hipLaunchKernelGGL((mixed_kernel<R, SIGN, NT, COL, POST>), dim3(grid), dim3(NT), slots * sizeof(cpx<R>), st,
+    hipLaunchKernelGGL((mixed_kernel<R, SIGN, NT, COL, POST, E>), dim3(grid), dim3(NT), slots * sizeof(cpx<R>), st,
                        static_cast<const cpx<R> *>(in), static_cast<cpx<R> *>(out), a);
 }
 
 template <typename R, int SIGN, int NT>
 static void launch_nt(const void *in, void *out, const MixedArgs &a, unsigned grid, hipStream_t st)
 {
+    if constexpr (NT == 1024 && sizeof(R) == 4)
+        if (a.e == MIXED_WIDE) {
+            if (a.pt_n) launch<R, SIGN, NT, true, true, MIXED_WIDE>(in, out, a, grid, st);
+            else launch<R, SIGN, NT, true, false, MIXED_WIDE>(in, out, a, grid, st);
+            return;
+        }
     const bool col = a.is != 1 || a.ois != 1;  // the planner's post-twiddle passes are strided
     if (a.pt_n) launch<R, SIGN, NT, true, true>(in, out, a, grid, st);
     else if (col) launch<R, SIGN, NT, true, false>(in, out, a, grid, st);

@@ -210,11 +210,10 @@ __device__ __forceinline__ void dft_mixed(cpx<R> (&x)[r])
     else dft<r, SIGN>(x);
 }
 
-// Registers: a thread holds up to MIXED_E elements, as 16 / r butterflies of
-// radix r (butterfly b, element m in v[b r + m]).
-constexpr int MIXED_E = 16;
-template <int r>
-constexpr int mixed_bf() { return MIXED_E / r; }
+// Registers: a thread holds up to E = MIXED_E elements (MIXED_WIDE in some
+// complex64 columns, see mixed_schedule), as E / r butterflies of radix r
+// (butterfly b, element m in v[b r + m]).
+constexpr int MIXED_E = 16, MIXED_WIDE = 32;
 
 // A stage of the block: radix-r butterfly bi < count is butterfly j of line
 // t; neighbouring lanes take neighbouring j (BYLINE false) or lines.
@@ -248,13 +247,13 @@ template <bool COL>
 __host__ __device__ __forceinline__ int mixed_slots(int n, int tb, int tbp) { return COL ? n * tbp : n * tb; }
 
 // LDS to registers and back.
-template <int r, typename R, int NT, bool COL>
-__device__ __forceinline__ void stage_get(cpx<R> (&v)[MIXED_E], const cpx<R> *lds, const Stage &st, int n, int tb,
+template <int r, typename R, int NT, bool COL, int E>
+__device__ __forceinline__ void stage_get(cpx<R> (&v)[E], const cpx<R> *lds, const Stage &st, int n, int tb,
                                           int tbp, const Div32 &dtb, int tid)
 {
     const int step = COL ? st.nb * tbp : st.nb;
 #pragma unroll
-    for (int b = 0; b < mixed_bf<r>(); ++b) {
+    for (int b = 0; b < E / r; ++b) {
         const int bi = tid + b * NT;
         if (bi < tb * st.nb) {
             int t, j;
@@ -266,13 +265,13 @@ __device__ __forceinline__ void stage_get(cpx<R> (&v)[MIXED_E], const cpx<R> *ld
     }
 }
 
-template <int r, typename R, int NT, bool COL>
-__device__ __forceinline__ void stage_put(const cpx<R> (&v)[MIXED_E], cpx<R> *lds, const Stage &st, int n, int tb,
+template <int r, typename R, int NT, bool COL, int E>
+__device__ __forceinline__ void stage_put(const cpx<R> (&v)[E], cpx<R> *lds, const Stage &st, int n, int tb,
                                           int tbp, const Div32 &dtb, bool byline, int tid)
 {
     const int step = COL ? st.Ns * tbp : st.Ns;
 #pragma unroll
-    for (int b = 0; b < mixed_bf<r>(); ++b) {
+    for (int b = 0; b < E / r; ++b) {
         const int bi = tid + b * NT;
         if (bi < tb * st.nb) {
             int t, j, kk;
@@ -290,12 +289,12 @@ __device__ __forceinline__ void stage_put(const cpx<R> (&v)[MIXED_E], cpx<R> *ld
 // ahead of the barrier that the stage's LDS reads wait behind.
 template <int r>
 constexpr int mixed_ntw() { return r <= 2 ? 1 : r <= 4 ? 2 : r <= 8 ? 3 : 4; }
-template <int r, typename R, int NT, bool COL>
-__device__ __forceinline__ void stage_tw(cpx<R> (&w)[mixed_bf<r>()][mixed_ntw<r>()], const Stage &st, int tb,
+template <int r, typename R, int NT, bool COL, int BF>
+__device__ __forceinline__ void stage_tw(cpx<R> (&w)[BF][mixed_ntw<r>()], const Stage &st, int tb,
                                          const Div32 &dtb, int tid)
 {
 #pragma unroll
-    for (int b = 0; b < mixed_bf<r>(); ++b) {
+    for (int b = 0; b < BF; ++b) {
         const int bi = tid + b * NT;
         if (bi < tb * st.nb) {
             int t, j, kk;
@@ -309,11 +308,11 @@ __device__ __forceinline__ void stage_tw(cpx<R> (&w)[mixed_bf<r>()][mixed_ntw<r>
 }
 
 // The butterflies of a stage, in registers; stage_run_tw with twiddles.
-template <int r, int SIGN, typename R, int NT>
-__device__ __forceinline__ void stage_run(cpx<R> (&v)[MIXED_E], const Stage &st, int tb, int tid)
+template <int r, int SIGN, typename R, int NT, int E>
+__device__ __forceinline__ void stage_run(cpx<R> (&v)[E], const Stage &st, int tb, int tid)
 {
 #pragma unroll
-    for (int b = 0; b < mixed_bf<r>(); ++b) {
+    for (int b = 0; b < E / r; ++b) {
         if (tid + b * NT < tb * st.nb) {
             cpx<R> x[r];
 #pragma unroll
@@ -324,12 +323,12 @@ __device__ __forceinline__ void stage_run(cpx<R> (&v)[MIXED_E], const Stage &st,
         }
     }
 }
-template <int r, int SIGN, typename R, int NT>
-__device__ __forceinline__ void stage_run_tw(cpx<R> (&v)[MIXED_E], const cpx<R> (&wt)[mixed_bf<r>()][mixed_ntw<r>()],
+template <int r, int SIGN, typename R, int NT, int E, int BF>
+__device__ __forceinline__ void stage_run_tw(cpx<R> (&v)[E], const cpx<R> (&wt)[BF][mixed_ntw<r>()],
                                              const Stage &st, int tb, int tid)
 {
 #pragma unroll
-    for (int b = 0; b < mixed_bf<r>(); ++b) {
+    for (int b = 0; b < BF; ++b) {
         if (tid + b * NT < tb * st.nb) {
             cpx<R> x[r], w[r];
 #pragma unroll
@@ -360,12 +359,12 @@ __device__ __forceinline__ void line_at(const Lines &g, int t, long long &o, lon
 
 // First stage (Ns = 1): the input lines to registers (a line past the last
 // reads the last one's elements; its results are not stored).
-template <int r, typename R, int NT>
-__device__ __forceinline__ void stage_load(cpx<R> (&v)[MIXED_E], const cpx<R> *in, const MixedArgs &a,
+template <int r, typename R, int NT, int E>
+__device__ __forceinline__ void stage_load(cpx<R> (&v)[E], const cpx<R> *in, const MixedArgs &a,
                                            const Lines &g, const Stage &st, const Div32 &dtb, bool byline, int tid)
 {
 #pragma unroll
-    for (int b = 0; b < mixed_bf<r>(); ++b) {
+    for (int b = 0; b < E / r; ++b) {
         const int bi = tid + b * NT;
         if (bi < a.tb * st.nb) {
             int t, j;
@@ -383,13 +382,13 @@ __device__ __forceinline__ void stage_load(cpx<R> (&v)[MIXED_E], const cpx<R> *i
 
 // Last stage (Ns r = n, so butterfly j writes j + m Ns): registers to the
 // output lines, scaled, with the four-step post-twiddle (POST).
-template <int r, int SIGN, typename R, int NT, bool POST>
-__device__ __forceinline__ void stage_store(cpx<R> (&v)[MIXED_E], cpx<R> *out, const MixedArgs &a,
+template <int r, int SIGN, typename R, int NT, bool POST, int E>
+__device__ __forceinline__ void stage_store(cpx<R> (&v)[E], cpx<R> *out, const MixedArgs &a,
                                             const Lines &g, const Stage &st, const Div32 &dtb, bool byline, int tid)
 {
     const R sc = (R)a.scale;
 #pragma unroll
-    for (int b = 0; b < mixed_bf<r>(); ++b) {
+    for (int b = 0; b < E / r; ++b) {
         const int bi = tid + b * NT;
         if (bi < a.tb * st.nb) {
             int t, j;
@@ -465,7 +464,7 @@ __device__ __forceinline__ int opaque_tid()
 // writes, barriers included (the radix is uniform), so that no registers
 // are live from one case to another: carried over the switches, the element
 // array spilled.
-template <typename R, int SIGN, int NT, bool COL, bool POST>
+template <typename R, int SIGN, int NT, bool COL, bool POST, int E>
 __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4)))
 mixed_kernel(const cpx<R> *in, cpx<R> *out, const MixedArgs a)
 {
@@ -491,7 +490,7 @@ mixed_kernel(const cpx<R> *in, cpx<R> *out, const MixedArgs a)
     const Stage first = stage(0);
 #define MIXED_FIRST(r)                                                          \
     {                                                                           \
-        cpx<R> v[MIXED_E]{};                                                    \
+        cpx<R> v[E]{};                                                    \
         const int tid = opaque_tid();                                           \
         stage_load<r, R, NT>(v, in, a, g, first, dtb, in_cols, tid);            \
         stage_run<r, SIGN, R, NT>(v, first, tb, tid);                           \
@@ -502,9 +501,9 @@ mixed_kernel(const cpx<R> *in, cpx<R> *out, const MixedArgs a)
         const Stage st = stage(s);
 #define MIXED_MID(r)                                                            \
     {                                                                           \
-        cpx<R> v[MIXED_E]{};                                                    \
+        cpx<R> v[E]{};                                                    \
         const int tid = opaque_tid();                                           \
-        cpx<R> w[mixed_bf<r>()][mixed_ntw<r>()]{};                              \
+        cpx<R> w[E / r][mixed_ntw<r>()]{};                              \
         stage_tw<r, R, NT, COL>(w, st, tb, dtb, tid);                           \
         __syncthreads();                                                        \
         stage_get<r, R, NT, COL>(v, lds, st, n, tb, tbp, dtb, tid);                  \
@@ -518,9 +517,9 @@ mixed_kernel(const cpx<R> *in, cpx<R> *out, const MixedArgs a)
         const Stage st = stage(a.nst - 1);
 #define MIXED_LAST(r)                                                           \
     {                                                                           \
-        cpx<R> v[MIXED_E]{};                                                    \
+        cpx<R> v[E]{};                                                    \
         const int tid = opaque_tid();                                           \
-        cpx<R> w[mixed_bf<r>()][mixed_ntw<r>()]{};                              \
+        cpx<R> w[E / r][mixed_ntw<r>()]{};                              \
         stage_tw<r, R, NT, COL>(w, st, tb, dtb, tid);                           \
         __syncthreads();                                                        \
         stage_get<r, R, NT, COL>(v, lds, st, n, tb, tbp, dtb, tid);                  \
@@ -620,7 +619,7 @@ mixed_real_kernel(const cpx<R> *in, cpx<R> *out, const MixedArgs a, const MixedR
     {                                                                     \
         cpx<R> v[MIXED_E]{};                                              \
         const int tid = opaque_tid();                                     \
-        cpx<R> tw[mixed_bf<r>()][mixed_ntw<r>()]{};                       \
+        cpx<R> tw[MIXED_E / r][mixed_ntw<r>()]{};                       \
         stage_tw<r, R, NT, false>(tw, st, tb, dtb, tid);                  \
         __syncthreads();                                                  \
         stage_get<r, R, NT, false>(v, lds, st, n, tb, tbp, dtb, tid);     \
@@ -636,7 +635,7 @@ mixed_real_kernel(const cpx<R> *in, cpx<R> *out, const MixedArgs a, const MixedR
     {                                                                     \
         cpx<R> v[MIXED_E]{};                                              \
         const int tid = opaque_tid();                                     \
-        cpx<R> tw[mixed_bf<r>()][mixed_ntw<r>()]{};                       \
+        cpx<R> tw[MIXED_E / r][mixed_ntw<r>()]{};                       \
         stage_tw<r, R, NT, false>(tw, st, tb, dtb, tid);                  \
         __syncthreads();                                                  \
         stage_get<r, R, NT, false>(v, lds, st, n, tb, tbp, dtb, tid);     \
