@@ -181,7 +181,10 @@ void topeFFTSynchronize(struct topeFFT *f);
  * launch at the position of chirp_pre), and per-launch timing:
  * while enabled, every Exec records HIP events around each launch on
  * f->stream; topePlanPassTimes synchronises and returns the mean duration
- * in milliseconds of each launch position over the recorded execs. */
+ * in milliseconds of each launch position over the recorded execs.
+ * topePlanExecPtr of one or more FP64 transforms of 2^24 points (a 1D or batch
+ * plan) runs a schedule of its own: count, names and times are those of the
+ * schedule that ran last since timing was switched on, of Exec's if none did. */
 int topePlanPassCount(void *plan_impl);
 void topePlanPassTiming(void *plan_impl, int enable);
 int topePlanPassTimes(struct topeFFT *f, void *plan_impl, double *ms, int max_passes);

@@ -1,0 +1,86 @@
+"""What the library asks of the HIP runtime, on the CPU: libtopefft.so in a
+process of its own with the runtime calls counted (hip_call_log.c), so kernel
+launches, copies and events of an entry point can be compared with what the
+library says of itself."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+PYDIR = os.path.join(os.path.dirname(HERE), "tope-fft_amd", "python")
+
+PRELUDE = """
+import ctypes as C, sys
+log = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
+sys.path.insert(0, sys.argv[2])
+import numpy as np
+import topefft
+F, B = topefft.FORWARD, topefft.INVERSE
+
+def launches(call):
+    before = log.log_launches()
+    call()
+    return log.log_launches() - before
+"""
+
+
+@pytest.fixture(scope="module")
+def run(tmp_path_factory):
+    import topefft
+    if not os.path.exists(topefft.LIB_PATH):
+        pytest.skip("libtopefft.so not built")
+    so = str(tmp_path_factory.mktemp("log") / "hip_call_log.so")
+    inc = os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "include")
+    subprocess.run(["gcc", "-shared", "-fPIC", "-O1", "-w", "-I", inc, "-o", so,
+                    os.path.join(HERE, "hip_call_log.c")], check=True)
+
+    def go(body):
+        r = subprocess.run([sys.executable, "-c", PRELUDE + body, so, PYDIR], capture_output=True, text=True,
+                           timeout=300)
+        assert r.returncode == 0, r.stderr[-2000:]
+        return r.stdout
+
+    return go
+
+
+# FP64 2^24 is the length whose callers' arrays run another schedule than the
+# plan's own array; 2^16 runs one with exchanged buffers, 4096 x 64 the same
+# passes in both
+@pytest.mark.parametrize("dims", [(1 << 24,), (1 << 16,), (4096, 64)], ids=lambda d: "x".join(map(str, d)))
+def test_pass_times_of_caller_array(run, dims):
+    """Names, count and times follow the schedule that the timed call ran."""
+    run(f"""
+dims = {dims!r}
+fw = topefft.Framework()
+p = topefft.Plan(fw, dims, np.zeros(int(np.prod(dims)), complex))
+own, data = p.pass_names(), p.t.data
+a = np.zeros(8, complex)
+ptr = a.ctypes.data // 16 * 16
+n_own, n_ptr = launches(lambda: p.exec_device(F)), launches(lambda: p.exec_ptr(ptr, F))
+p.pass_timing(True)
+for _ in range(3):
+    assert launches(lambda: p.exec_ptr(ptr, F)) == n_ptr
+ms, names = p.pass_times(), p.pass_names()
+assert len(ms) == len(names) == p.pass_count() == n_ptr, (ms, names)
+assert list(ms) == [1.0] * n_ptr, ms
+# both schedules in one recording: the last one's times alone
+p.exec_ptr(ptr, B)
+assert launches(lambda: p.exec_device(F)) == n_own
+assert p.pass_names() == own
+assert list(p.pass_times()) == [1.0] * n_own
+p.exec_device(F)
+p.exec_ptr(ptr, F)
+assert list(p.pass_times()) == [1.0] * n_ptr
+for i in range(n_ptr):
+    assert p.time_pass(i, F, 4) == 1.0
+# switched on again: the plan's own schedule until a transform is timed
+p.pass_timing(False)
+p.pass_timing(True)
+assert p.pass_names() == own and list(p.pass_times()) == [0.0] * n_own
+p.pass_timing(False)
+p.exec_ptr(ptr, F)
+assert p.pass_names() == own
+p.destroy()
+""")

@@ -162,6 +162,7 @@ struct PlanImpl {
     int alt_pass = -1;
     bool alternate = false;
     std::vector<Pass> ptr_passes;
+    bool caller_list = false;  // `passes` holds ptr_passes for the length of a call (CallerList)
     std::vector<void *> allocs;
     std::map<std::pair<int, int>, void *> stage_tw;  // (n, e + 64 * prec) -> table
     struct AxisTw {
@@ -178,11 +179,46 @@ struct PlanImpl {
     std::vector<int> inv_order;
     bool real_scratch0 = false;  // a column pass uses buffer 0 (P->bytes) as scratch
     EventPair run;  // this plan's exec events
-    // per-pass timing
+    // per-pass timing: what was timed since the last topePlanPassTimes
     bool timing = false;
+    bool timed_caller_list = false;  // the last timed transform ran ptr_passes
     std::vector<hipEvent_t> pool;
     size_t pool_used = 0;
-    std::vector<std::pair<int, std::pair<hipEvent_t, hipEvent_t>>> pending;
+    struct Timed {
+        int pass;  // position in its schedule
+        bool caller_list;
+        hipEvent_t start, stop;
+    };
+    std::vector<Timed> pending;
+};
+
+// The schedule whose positions the pass queries describe: the one that the
+// last timed transform ran, else the plan's own.
+const std::vector<Pass> &listed_passes(const PlanImpl *P)
+{
+    return P->timed_caller_list ? P->ptr_passes : P->passes;
+}
+
+// While one lives, `passes` is the callers' schedule, which ends in buffer 0.
+struct CallerList {
+    PlanImpl *P;
+    int final_buf;
+    explicit CallerList(PlanImpl *plan, bool on) : P(on ? plan : nullptr), final_buf(plan->final_buf)
+    {
+        if (!P) return;
+        P->passes.swap(P->ptr_passes);
+        P->final_buf = 0;
+        P->caller_list = true;
+    }
+    ~CallerList()
+    {
+        if (!P) return;
+        P->passes.swap(P->ptr_passes);
+        P->final_buf = final_buf;
+        P->caller_list = false;
+    }
+    CallerList(const CallerList &) = delete;
+    CallerList &operator=(const CallerList &) = delete;
 };
 
 thread_local std::string g_msg;
@@ -1268,6 +1304,7 @@ int enqueue(PlanImpl *P, hipStream_t s, int dir)
 {
     if (dir != FORWARD && dir != INVERSE) return TOPE_ERROR_INVALID_ARG;
     const bool rev = dir == INVERSE && !P->inv_order.empty();
+    if (P->timing) P->timed_caller_list = P->caller_list;
     for (size_t n = 0; n < P->passes.size(); ++n) {
         const size_t i = rev ? (size_t)P->inv_order[n] : n;
         hipEvent_t e0 = nullptr, e1 = nullptr;
@@ -1293,7 +1330,7 @@ int enqueue(PlanImpl *P, hipStream_t s, int dir)
         if (rc) return rc;
         if (P->timing) {
             (void)hipEventRecord(e1, s);
-            P->pending.push_back({(int)i, {e0, e1}});
+            P->pending.push_back({(int)i, P->caller_list, e0, e1});
         }
     }
     if (P->final_buf == 1 && !P->alternate) std::swap(P->buf[0], P->buf[1]);
@@ -2357,13 +2394,14 @@ void topeFFTSynchronize(struct topeFFT *f)
 int topePlanPassCount(void *plan_impl)
 {
     PlanImpl *P = impl_of(plan_impl);
-    return P ? (int)P->passes.size() : 0;
+    return P ? (int)listed_passes(P).size() : 0;
 }
 
 void topePlanPassTiming(void *plan_impl, int enable)
 {
     PlanImpl *P = impl_of(plan_impl);
     if (!P) return;
+    if (enable && !P->timing) P->timed_caller_list = false;
     P->timing = enable != 0;
     if (!P->timing) {
         P->pending.clear();
@@ -2384,14 +2422,15 @@ int topePlanPassTimes(struct topeFFT *f, void *plan_impl, double *ms, int max_pa
         f->error = map_err(err);
         return 0;
     }
-    const int np = (int)P->passes.size();
+    const int np = (int)listed_passes(P).size();
     std::vector<double> sum(np, 0.0);
     std::vector<long long> cnt(np, 0);
-    for (auto &pe : P->pending) {
+    for (const PlanImpl::Timed &pe : P->pending) {
+        if (pe.caller_list != P->timed_caller_list) continue;  // positions of the other schedule
         float t = 0;
-        if (hipEventElapsedTime(&t, pe.second.first, pe.second.second) == hipSuccess) {
-            sum[pe.first] += t;
-            cnt[pe.first]++;
+        if (hipEventElapsedTime(&t, pe.start, pe.stop) == hipSuccess) {
+            sum[pe.pass] += t;
+            cnt[pe.pass]++;
         }
     }
     P->pending.clear();
@@ -2406,11 +2445,12 @@ double topePlanTimePass(struct topeFFT *f, void *plan_impl, int pass, int dir, i
 {
     PlanImpl *P = impl_of(plan_impl);
     FrameworkImpl *fw = fw_of(f);
-    if (!P || !fw || pass < 0 || pass >= (int)P->passes.size() || reps < 1 ||
+    if (!P || !fw || pass < 0 || pass >= (int)listed_passes(P).size() || reps < 1 ||
         (dir != FORWARD && dir != INVERSE)) {
         if (f) f->error = TOPE_ERROR_INVALID_ARG;
         return -1.0;
     }
+    const CallerList list(P, P->timed_caller_list);
     EventPair ev;
     hipError_t err = time_start(ev, fw->stream, false);
     int rc = TOPE_SUCCESS;
@@ -2426,8 +2466,8 @@ double topePlanTimePass(struct topeFFT *f, void *plan_impl, int pass, int dir, i
 const char *topePlanPassName(void *plan_impl, int pass)
 {
     PlanImpl *P = impl_of(plan_impl);
-    if (!P || pass < 0 || pass >= (int)P->passes.size()) return "";
-    return P->passes[pass].name;
+    if (!P || pass < 0 || pass >= (int)listed_passes(P).size()) return "";
+    return listed_passes(P)[pass].name;
 }
 
 /* ---- real-input transforms (no reference counterpart) ------------------- */
@@ -2614,20 +2654,11 @@ void topePlanExecPtr(struct topeFFT *f, void *plan_impl, void *data, int dir)
     // 16.5 us, 2^16 22.6 -> 16.5 us, 2^20 64 -> 41 us, 2^24 882 -> 645 us
     void *own0 = P->buf[0], *own1 = P->buf[1];
     P->buf[0] = data;
-    const int final_buf = P->final_buf;
-    const bool own_list = !P->ptr_passes.empty();
-    P->alternate = !own_list && P->alt_pass >= 0;
-    if (own_list) {
-        P->passes.swap(P->ptr_passes);
-        P->final_buf = 0;
-    }
+    const CallerList list(P, !P->ptr_passes.empty());
+    P->alternate = !P->caller_list && P->alt_pass >= 0;
     int rc = enqueue(P, fw->stream, dir);
     const bool copy = P->final_buf == 1 && !P->alternate;
     P->alternate = false;
-    if (own_list) {
-        P->passes.swap(P->ptr_passes);
-        P->final_buf = final_buf;
-    }
     if (!rc && copy)
         rc = map_err(hipMemcpyAsync(data, P->buf[0], P->bytes, hipMemcpyDeviceToDevice, fw->stream));
     P->buf[0] = own0;
