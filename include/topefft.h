@@ -176,25 +176,29 @@ void topePlanDownload(struct topeFFT *f, void *plan_impl, void *host, size_t byt
 /* Wait for all work enqueued on f->stream. */
 void topeFFTSynchronize(struct topeFFT *f);
 
-/* Number of kernel launches one Exec performs (a length with a prime factor
- * above 7 and at most 2048 counts chirp_pre and chirp_post, which share one
- * launch at the position of chirp_pre), and per-launch timing:
- * while enabled, every Exec records HIP events around each launch on
- * f->stream; topePlanPassTimes synchronises and returns the mean duration
- * in milliseconds of each launch position over the recorded execs.
+/* Number of passes of one Exec, and per-pass timing.  A pass is one kernel
+ * launch at its position, but for
+ *   - 3D arrays of 512 MiB and more: their X and Y passes take turns over
+ *     chunks of planes, one launch of each for a chunk;
+ *   - a length with a prime factor above 7 and at most 2048: chirp_pre and
+ *     chirp_post share one launch at the position of chirp_pre;
+ *   - a few axes of three strides, whose pass repeats its launch.
+ * While timing is enabled, every Exec records HIP events around each launch on
+ * f->stream; topePlanPassTimes synchronises and returns for each pass the mean
+ * time in milliseconds that its launches took in one of the recorded execs.
  * topePlanExecPtr of one or more FP64 transforms of 2^24 points (a 1D or batch
  * plan) runs a schedule of its own: count, names and times are those of the
  * schedule that ran last since timing was switched on, of Exec's if none did. */
 int topePlanPassCount(void *plan_impl);
 void topePlanPassTiming(void *plan_impl, int enable);
 int topePlanPassTimes(struct topeFFT *f, void *plan_impl, double *ms, int max_passes);
-/* Mean device time in milliseconds of launch position `pass` alone: HIP
- * events around `reps` back-to-back launches of that pass on f->stream (no
+/* Mean device time in milliseconds of pass `pass` alone: HIP
+ * events around `reps` back-to-back runs of that pass over the whole array on f->stream (no
  * events between the launches).  Repeating one pass in isolation leaves the
  * plan's device data in an undefined state: upload again before the next
  * transform whose result matters. */
 double topePlanTimePass(struct topeFFT *f, void *plan_impl, int pass, int dir, int reps);
-/* Kernel name of launch position `pass` (static string). */
+/* Kernel name of pass `pass` (static string). */
 const char *topePlanPassName(void *plan_impl, int pass);
 
 /* ---- batched 1D transforms (no reference counterpart) -------------------

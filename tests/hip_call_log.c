@@ -17,7 +17,16 @@ static long launches, copies;
 static unsigned last_flags[4096];
 static int records;
 
+static unsigned long sequence;
+
 long log_launches(void) { return launches; }
+/* Stands for the kernels launched since the last call, in their order. */
+unsigned long log_sequence(void)
+{
+    const unsigned long s = sequence;
+    sequence = 0;
+    return s;
+}
 long log_copies(void) { return copies; }
 /* Events recorded since the last call: their creation flags. */
 int log_records(unsigned *flags, int max)
@@ -52,6 +61,7 @@ hipError_t __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *m, hipStream_t *s
 hipError_t hipLaunchKernel(const void *f, dim3 g, dim3 b, void **a, size_t m, hipStream_t s)
 {
     ++launches;
+    sequence = sequence * 1000003 + (unsigned long)f;
     return hipSuccess;
 }
 

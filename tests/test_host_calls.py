@@ -18,11 +18,18 @@ sys.path.insert(0, sys.argv[2])
 import numpy as np
 import topefft
 F, B = topefft.FORWARD, topefft.INVERSE
+log.log_launches.restype = C.c_long
+log.log_sequence.restype = C.c_ulong
 
 def launches(call):
     before = log.log_launches()
     call()
     return log.log_launches() - before
+
+def sequence(call):
+    log.log_sequence()
+    call()
+    return log.log_sequence()
 """
 
 
@@ -82,5 +89,41 @@ assert p.pass_names() == own and list(p.pass_times()) == [0.0] * n_own
 p.pass_timing(False)
 p.exec_ptr(ptr, F)
 assert p.pass_names() == own
+p.destroy()
+""")
+
+
+# 3D arrays of 512 MiB and more run their X and Y passes over chunks of
+# planes: complex64 512 x 512 x 256 in two, FP64 512^3 in eight, a real array
+# whose inverse runs the chunks last; 64 x 32 x 16 is not chunked
+@pytest.mark.parametrize("kind,dims,chunks", [("f32", (512, 512, 256), 2), ("f64", (512, 512, 512), 8),
+                                              ("real", (1024, 512, 256), 8), ("f64", (64, 32, 16), 1)],
+                         ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
+def test_timed_transforms_make_the_same_launches(run, kind, dims, chunks):
+    """Timing changes nothing of the schedule, and a pass's time is the sum of its launches."""
+    run(f"""
+kind, dims, chunks = {kind!r}, {dims!r}, {chunks!r}
+fw = topefft.Framework()
+n = int(np.prod(dims))
+if kind == "real":
+    p = topefft.RealPlan(fw, dims, np.zeros(n))
+    impl = p.t.impl
+elif kind == "f32":
+    p = topefft.Plan(fw, dims, np.zeros(n, np.complex64), precision=topefft.PREC_F32)
+    impl = p.impl
+else:
+    p = topefft.Plan(fw, dims, np.zeros(n, complex))
+    impl = p.impl
+ms = (C.c_double * 8)()
+for d in (F, B):
+    assert launches(lambda: p.exec_device(d)) == 2 * chunks + 1
+    want = sequence(lambda: p.exec_device(d))
+    fw.lib.topePlanPassTiming(impl, 1)
+    for _ in range(3):
+        assert sequence(lambda: p.exec_device(d)) == want
+    got = fw.lib.topePlanPassTimes(C.byref(fw.f), impl, ms, 8)
+    fw.lib.topePlanPassTiming(impl, 0)
+    assert got == p.pass_count() == 3
+    assert sorted(ms[:3]) == [1, chunks, chunks], ms[:3]
 p.destroy()
 """)

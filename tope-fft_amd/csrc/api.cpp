@@ -187,6 +187,7 @@ struct PlanImpl {
     struct Timed {
         int pass;  // position in its schedule
         bool caller_list;
+        bool first;  // the pass's first launch of a transform (a chunked pass has several)
         hipEvent_t start, stop;
     };
     std::vector<Timed> pending;
@@ -1305,33 +1306,31 @@ int enqueue(PlanImpl *P, hipStream_t s, int dir)
     if (dir != FORWARD && dir != INVERSE) return TOPE_ERROR_INVALID_ARG;
     const bool rev = dir == INVERSE && !P->inv_order.empty();
     if (P->timing) P->timed_caller_list = P->caller_list;
-    for (size_t n = 0; n < P->passes.size(); ++n) {
-        const size_t i = rev ? (size_t)P->inv_order[n] : n;
-        hipEvent_t e0 = nullptr, e1 = nullptr;
-        if (P->timing) {
-            e0 = pool_event(P);
-            e1 = pool_event(P);
-            if (!e0 || !e1) return TOPE_ERROR_UNSUPPORTED;
-            (void)hipEventRecord(e0, s);
-        }
-        int rc = TOPE_SUCCESS;
-        if (P->passes[i].group && !P->timing) {
-            // the group's passes chunk by chunk
-            const int g = P->passes[i].group;
-            size_t e = n;
-            while (e < P->passes.size() && P->passes[rev ? (size_t)P->inv_order[e] : e].group == g) ++e;
-            for (long long r = 0; r < P->passes[i].reps && !rc; ++r)
-                for (size_t k = n; k < e && !rc; ++k)
-                    rc = launch_pass(P, rev ? (size_t)P->inv_order[k] : k, s, dir, r, r + 1);
-            n = e - 1;
-        } else {
-            rc = launch_pass(P, i, s, dir);
-        }
+    auto at = [&](size_t n) { return rev ? (size_t)P->inv_order[n] : n; };
+    auto launch = [&](size_t i, long long rep0, long long rep1) -> int {
+        if (!P->timing) return launch_pass(P, i, s, dir, rep0, rep1);
+        hipEvent_t e0 = pool_event(P), e1 = pool_event(P);
+        if (!e0 || !e1) return TOPE_ERROR_UNSUPPORTED;
+        (void)hipEventRecord(e0, s);
+        const int rc = launch_pass(P, i, s, dir, rep0, rep1);
         if (rc) return rc;
-        if (P->timing) {
-            (void)hipEventRecord(e1, s);
-            P->pending.push_back({(int)i, P->caller_list, e0, e1});
+        (void)hipEventRecord(e1, s);
+        P->pending.push_back({(int)i, P->caller_list, rep0 == 0, e0, e1});
+        return TOPE_SUCCESS;
+    };
+    for (size_t n = 0; n < P->passes.size(); ++n) {
+        const Pass &ps = P->passes[at(n)];
+        if (!ps.group) {
+            if (int rc = launch(at(n), 0, -1)) return rc;
+            continue;
         }
+        // the group's passes chunk by chunk
+        size_t e = n;
+        while (e < P->passes.size() && P->passes[at(e)].group == ps.group) ++e;
+        for (long long r = 0; r < ps.reps; ++r)
+            for (size_t k = n; k < e; ++k)
+                if (int rc = launch(at(k), r, r + 1)) return rc;
+        n = e - 1;
     }
     if (P->final_buf == 1 && !P->alternate) std::swap(P->buf[0], P->buf[1]);
     return TOPE_SUCCESS;
@@ -2430,7 +2429,7 @@ int topePlanPassTimes(struct topeFFT *f, void *plan_impl, double *ms, int max_pa
         float t = 0;
         if (hipEventElapsedTime(&t, pe.start, pe.stop) == hipSuccess) {
             sum[pe.pass] += t;
-            cnt[pe.pass]++;
+            cnt[pe.pass] += pe.first;
         }
     }
     P->pending.clear();
