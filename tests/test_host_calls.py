@@ -127,3 +127,30 @@ for d in (F, B):
     assert sorted(ms[:3]) == [1, chunks, chunks], ms[:3]
 p.destroy()
 """)
+
+
+@pytest.mark.parametrize("order", ["small first", "large first"])
+def test_exec_event_fences(run, order):
+    """An Exec of up to 256 KiB records its transform with events that have no
+    system-scope fence and a fenced one behind its copy, a larger Exec fenced ones
+    throughout, whichever the framework ran first; profileThis reads the last one's."""
+    run(f"""
+fw = topefft.Framework()
+small = topefft.Plan(fw, (1024,), np.zeros(1024, complex))
+large = topefft.Plan(fw, (1 << 16,), np.zeros(1 << 16, complex))
+PLAIN, FENCED = 0x20000000, 0  # hipEventDisableSystemFence, hipEventDefault
+flags = (C.c_uint * 64)()
+
+def events(p):
+    log.log_records(flags, 64)
+    p.exec(F)
+    return list(flags[:log.log_records(flags, 64)])
+
+want = {{"small": [PLAIN, PLAIN, FENCED], "large": [FENCED] * 4}}
+for who in {["small", "large", "small", "large"] if order == "small first" else ["large", "small", "large", "small"]!r}:
+    p = small if who == "small" else large
+    assert events(p) == want[who], (who, flags[:4])
+    assert fw.lib.profileThis(fw.f.event) == 1e6 * p.pass_count()  # a launch counts a millisecond
+small.destroy()
+large.destroy()
+""")

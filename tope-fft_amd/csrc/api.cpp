@@ -44,11 +44,24 @@ struct EventPair {
     bool recorded = false;
 };
 
+// Device times of execs: a pair that the general path brackets a transform
+// with before a host copy reads it, and one for execs that record a fenced event
+// of their own behind their copy (ensure_event on the fence).
+struct LastExec {
+    EventPair fenced, plain;
+    EventPair *latest = nullptr;
+    EventPair &next(bool fence)
+    {
+        latest = fence ? &fenced : &plain;
+        return *latest;
+    }
+};
+
 struct FrameworkImpl {
     hipStream_t stream = nullptr;  // the stream every plan op is enqueued on
     hipStream_t own = nullptr;     // the framework's own stream (stream unless a caller's is set)
     int live_plans = 0;
-    EventPair last;  // last exec's device time (profileThis)
+    LastExec last;  // last exec's device time (profileThis)
     hipEvent_t copied = nullptr;  // behind the download of the last small exec
     bool stage_ref = false;       // this framework holds a reference to the staging buffer
 };
@@ -1860,8 +1873,10 @@ void release_framework(struct topeFFT *f)
         (void)hipStreamSynchronize(fw->own);
         (void)hipStreamDestroy(fw->own);
     }
-    if (fw->last.start) (void)hipEventDestroy(fw->last.start);
-    if (fw->last.stop) (void)hipEventDestroy(fw->last.stop);
+    for (const EventPair *ev : {&fw->last.fenced, &fw->last.plain}) {
+        if (ev->start) (void)hipEventDestroy(ev->start);
+        if (ev->stop) (void)hipEventDestroy(ev->stop);
+    }
     if (fw->copied) (void)hipEventDestroy(fw->copied);
     stage_release(fw);
     delete fw;
@@ -1884,19 +1899,20 @@ double elapsed_ns(hipEvent_t a, hipEvent_t b)
 int exec_staged(FrameworkImpl *fw, PlanImpl *P, void *stage, void *d, int dir, tope_ulong *kern_ns, tope_ulong *mem_ns)
 {
     hipStream_t s = fw->stream;
+    EventPair &ev = fw->last.next(false);
     hipError_t err = ensure_event(&fw->copied);
-    if (err == hipSuccess) err = time_start(fw->last, s, false);
+    if (err == hipSuccess) err = time_start(ev, s, false);
     if (err != hipSuccess) return map_err(err);
     const int rc = enqueue(P, s, dir);
     if (rc) return rc;
-    err = time_stop(fw->last, s, nullptr);
+    err = time_stop(ev, s, nullptr);
     if (err == hipSuccess) err = copy_out(P->buf[0], stage, P->bytes, s);
     if (err == hipSuccess) err = hipEventRecord(fw->copied, s);
     if (err == hipSuccess) err = hipEventSynchronize(fw->copied);
     if (err != hipSuccess) return map_err(err);
     std::memcpy(d, stage, P->bytes);
-    *kern_ns += (tope_ulong)elapsed_ns(fw->last.start, fw->last.stop);
-    *mem_ns += (tope_ulong)elapsed_ns(fw->last.stop, fw->copied);
+    *kern_ns += (tope_ulong)elapsed_ns(ev.start, ev.stop);
+    *mem_ns += (tope_ulong)elapsed_ns(ev.stop, fw->copied);
     return TOPE_SUCCESS;
 }
 
@@ -1914,11 +1930,12 @@ int exec_host(struct topeFFT *f, PlanImpl *P, void *d, int dir, tope_ulong *kern
         }
     }
     hipStream_t s = fw->stream;
-    hipError_t err = time_start(fw->last, s);
+    EventPair &ev = fw->last.next(true);
+    hipError_t err = time_start(ev, s);
     if (err != hipSuccess) return map_err(err);
     int rc = enqueue(P, s, dir);
     if (rc) return rc;
-    err = time_stop(fw->last, s, kern_ns);
+    err = time_stop(ev, s, kern_ns);
     if (err != hipSuccess) return map_err(err);
     EventPair dn;
     err = time_start(dn, s);
@@ -2031,7 +2048,8 @@ void topeFFTDestroy(struct topeFFT *f)
 
 tope_ulong profileThis(void *event)
 {
-    EventPair *ev = static_cast<EventPair *>(event);
+    const LastExec *last = static_cast<const LastExec *>(event);
+    const EventPair *ev = last ? last->latest : nullptr;
     if (!ev || !ev->recorded) return 0;
     if (hipEventSynchronize(ev->stop) != hipSuccess) return 0;
     float ms = 0;
@@ -2517,9 +2535,10 @@ void topeRealExecEx(struct topeFFT *f, struct topePlanReal *t, void *host, int d
         return;
     }
     hipStream_t s = fw->stream;
-    hipError_t err = time_start(fw->last, s);
+    EventPair &ev = fw->last.next(true);
+    hipError_t err = time_start(ev, s);
     int rc = err == hipSuccess ? enqueue(P, s, dir) : map_err(err);
-    if (!rc) rc = map_err(time_stop(fw->last, s, &t->totalKernel));
+    if (!rc) rc = map_err(time_stop(ev, s, &t->totalKernel));
     if (!rc) {
         EventPair dn;
         err = time_start(dn, s);
