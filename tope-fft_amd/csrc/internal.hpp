@@ -105,6 +105,7 @@ enum { CHIRP_FILTER = 0, CHIRP_PRE = 1, CHIRP_MUL = 2, CHIRP_POST = 3 };
 // o os + c cs, its elements are `is` apart.
 constexpr int MIXED_MAX_N = 4096;
 constexpr int MIXED_MAX_STAGES = 8;
+constexpr int MIXED_ROWS = 64;  // rows and threads of a block of packed rows of at most 16 points
 struct MixedStage {
     int r, nb, Ns;  // radix, butterflies per line, span
     int tw;         // first entry of the stage in the table

@@ -94,6 +94,13 @@ MixedArgs mixed_plan(long long n, long long O, long long os, long long C, long l
     return a;
 }
 
+// Contiguous lines back to back, in and out.
+static bool packed_rows(const MixedArgs &a)
+{
+    return a.is == 1 && a.ois == 1 && !a.pt_n && (a.C == 1 || (a.cs == a.n && a.ocs == a.n)) &&
+           (a.O == 1 || (a.os == a.C * a.n && a.oos == a.C * a.n));
+}
+
 void mixed_schedule(MixedArgs &a, int prec)
 {
     std::vector<int> rad = mixed_radices(a.n);
@@ -141,8 +148,7 @@ void mixed_schedule(MixedArgs &a, int prec)
         }
     };
     if (a.nst == 1) {
-        a.nt = 256;
-        a.tb = 256;
+        a.nt = a.tb = packed_rows(a) ? MIXED_ROWS : 256;
     } else {
         tile(MIXED_E, a.cap, 256, 64);
         // complex64 columns of which 1024 threads hold fewer than four at 16
@@ -216,7 +222,7 @@ hipError_t launch_mixed(int prec, const void *in, void *out, const MixedArgs &a,
     if (grid < 1 || grid > 0x7fffffffLL || a.nst < 1 || a.nst > MIXED_MAX_STAGES || a.tb < 1 ||
         (long long)a.tb * a.n > (long long)a.nt * a.cap || (a.nst > 1 && bytes > MIXED_LDS) ||
         (a.nt > 512 && !col) || (a.e != MIXED_E && (a.nt != 1024 || !col || prec != PREC_F32)) ||
-        (col && a.nst > 1 && a.tbp < a.tb) || (a.pt_n && !col && a.nst > 1))
+        (col && a.nst > 1 && a.tbp < a.tb) || (a.nst == 1 && a.nt != (packed_rows(a) ? MIXED_ROWS : 256)) || (a.pt_n && !col && a.nst > 1))
         return hipErrorInvalidValue;
     const unsigned g = (unsigned)grid;
     if (prec == PREC_F64)

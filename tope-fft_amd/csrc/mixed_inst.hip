@@ -33,7 +33,10 @@ hipError_t launch_mixed_t(const void *in, void *out, const MixedArgs &a, unsigne
     if (a.nst == 1) {
         const cpx<R> *i = static_cast<const cpx<R> *>(in);
         cpx<R> *o = static_cast<cpx<R> *>(out);
-        if (a.pt_n) hipLaunchKernelGGL((mixed_one_kernel<R, SIGN, true>), dim3(grid), dim3(256), 0, st, i, o, a);
+        if (a.nt == MIXED_ROWS)
+            hipLaunchKernelGGL((mixed_rows_kernel<R, SIGN>), dim3(grid), dim3(MIXED_ROWS),
+                               (size_t)MIXED_ROWS * (a.n | 1) * sizeof(cpx<R>), st, i, o, a);
+        else if (a.pt_n) hipLaunchKernelGGL((mixed_one_kernel<R, SIGN, true>), dim3(grid), dim3(256), 0, st, i, o, a);
         else hipLaunchKernelGGL((mixed_one_kernel<R, SIGN, false>), dim3(grid), dim3(256), 0, st, i, o, a);
         return hipGetLastError();
     }
