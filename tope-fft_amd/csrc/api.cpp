@@ -903,6 +903,9 @@ class Planner {
         ps.chirp_tab[0] = tab[0];
         ps.chirp_tab[1] = tab[1];
         ps.cl.g = ChirpGeo{g.O, g.os, g.C, g.cs, g.is};
+        // a block takes lines of one o: planes of a single column, whose lines are
+        // contiguous, count as one run of rows (1 x 11 x 50000: 263 -> 71 us)
+        if (g.C == 1) ps.cl.g = ChirpGeo{1, 0, g.O, g.os, g.is};
         ps.cl.n = (int)n;
         ps.cl.M = (int)M;
         ps.cl.chirp = ct;
