@@ -33,3 +33,13 @@ def test_planes_of_one_column(dims):
     """The middle axis lies along contiguous memory; the planes' lines share blocks of
     32 (11 and 13 points), 8 (127), 2 (509) and 1 (2039)."""
     _check(dims)
+
+
+# 16-line tiles for 32 < 2n - 1 <= 256 points of convolution, 8-line ones up to
+# 512, from 512 tiles on: 515 tiles, the last one half full; one width above:
+# full tiles and a partial one of 4 lines (509 points) or 2 (1021, 2039)
+@pytest.mark.parametrize("dims", [(8232, 31), (8232, 61), (8232, 127), (4116, 251), (35, 509), (2058, 509),
+                                  (35, 1021), (1029, 1021), (35, 2039), (1029, 2039), (12, 61, 25)],
+                         ids=lambda d: "x".join(map(str, d)))
+def test_column_tiles(dims):
+    _check(dims)

@@ -307,8 +307,13 @@ static hipError_t launch_line_t(const void *in, void *out, ChirpLineArgs a, hipS
 }
 
 // Rows: 64 to 256 threads a block.  Strided axes: tiles of WIDE adjacent
-// lines (64-byte segments or more), or NARROW ones where the wide tiles
-// would leave CUs with no more than one block.
+// lines, or NARROW ones where the wide tiles would leave CUs with no more than
+// one block.  Up to M = 512 wide tiles gain a little (4096 x 251: 51.9 us, 53.8
+// narrow; 8192 x 127 58.1 and 60.8); longer lines take one width, as more
+// blocks of fewer waves hide their serial stages better than wider segments
+// help: 4096 x 509 82 us in four lines, 90 in eight; 4096 x 1021 151 in two,
+// 180 in four; 4096 x 2039 343 in two, 373 in four, whose 1024 threads leave
+// 128 registers each and spill 24 (forward and inverse).
 template <int N, int ROW, int WIDE, int NARROW>
 static hipError_t launch_line_n(const void *in, void *out, const ChirpLineArgs &a, hipStream_t st)
 {
@@ -326,9 +331,9 @@ hipError_t launch_chirp_lines(const void *in, void *out, const ChirpLineArgs &a,
     case 128: return launch_line_n<128, 16, 16, 8>(in, out, a, st);
     case 256: return launch_line_n<256, 8, 16, 4>(in, out, a, st);
     case 512: return launch_line_n<512, 4, 8, 4>(in, out, a, st);
-    case 1024: return launch_line_n<1024, 2, 8, 4>(in, out, a, st);
-    case 2048: return launch_line_n<2048, 1, 4, 2>(in, out, a, st);
-    case 4096: return launch_line_n<4096, 1, 4, 2>(in, out, a, st);
+    case 1024: return launch_line_n<1024, 2, 4, 4>(in, out, a, st);
+    case 2048: return launch_line_n<2048, 1, 2, 2>(in, out, a, st);
+    case 4096: return launch_line_n<4096, 1, 2, 2>(in, out, a, st);
     default: return hipErrorInvalidValue;
     }
 }
