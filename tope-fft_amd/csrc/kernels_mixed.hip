@@ -222,7 +222,8 @@ hipError_t launch_mixed(int prec, const void *in, void *out, const MixedArgs &a,
     if (grid < 1 || grid > 0x7fffffffLL || a.nst < 1 || a.nst > MIXED_MAX_STAGES || a.tb < 1 ||
         (long long)a.tb * a.n > (long long)a.nt * a.cap || (a.nst > 1 && bytes > MIXED_LDS) ||
         (a.nt > 512 && !col) || (a.e != MIXED_E && (a.nt != 1024 || !col || prec != PREC_F32)) ||
-        (col && a.nst > 1 && a.tbp < a.tb) || (a.nst == 1 && a.nt != (packed_rows(a) ? MIXED_ROWS : 256)) || (a.pt_n && !col && a.nst > 1))
+        (col && a.nst > 1 && a.tbp < a.tb) || (a.nst == 1 && a.nt != (packed_rows(a) ? MIXED_ROWS : 256)) ||
+        (a.pt_n && (!col || a.nst == 1)))
         return hipErrorInvalidValue;
     const unsigned g = (unsigned)grid;
     if (prec == PREC_F64)

@@ -36,12 +36,11 @@ hipError_t launch_mixed_t(const void *in, void *out, const MixedArgs &a, unsigne
         if (a.nt == MIXED_ROWS)
             hipLaunchKernelGGL((mixed_rows_kernel<R, SIGN>), dim3(grid), dim3(MIXED_ROWS),
                                (size_t)MIXED_ROWS * (a.n | 1) * sizeof(cpx<R>), st, i, o, a);
-        else if (a.pt_n) hipLaunchKernelGGL((mixed_one_kernel<R, SIGN, true>), dim3(grid), dim3(256), 0, st, i, o, a);
-        else hipLaunchKernelGGL((mixed_one_kernel<R, SIGN, false>), dim3(grid), dim3(256), 0, st, i, o, a);
+        else
+            hipLaunchKernelGGL((mixed_one_kernel<R, SIGN>), dim3(grid), dim3(256), 0, st, i, o, a);
         return hipGetLastError();
     }
     switch (a.nt) {
-    case 128: launch_nt<R, SIGN, 128>(in, out, a, grid, st); break;
     case 256: launch_nt<R, SIGN, 256>(in, out, a, grid, st); break;
     case 512: launch_nt<R, SIGN, 512>(in, out, a, grid, st); break;
     case 1024: launch_nt<R, SIGN, 1024>(in, out, a, grid, st); break;

@@ -672,8 +672,9 @@ mixed_real_kernel(const cpx<R> *in, cpx<R> *out, const MixedArgs a, const MixedR
     }
 }
 
-// n <= 16: a radix of its own, one thread per line, no LDS.
-template <typename R, int SIGN, bool POST>
+// n <= 16: a radix of its own, one thread per line, no LDS.  (The factors of a
+// four-step are never that short: 35 points is the least of any length.)
+template <typename R, int SIGN>
 __global__ void __launch_bounds__(256) mixed_one_kernel(const cpx<R> *in, cpx<R> *out, const MixedArgs a)
 {
     const Div32 dtb{a.tb, a.inv_tb};
@@ -691,7 +692,7 @@ __global__ void __launch_bounds__(256) mixed_one_kernel(const cpx<R> *in, cpx<R>
         const int tid = opaque_tid();                                           \
         stage_load<r, R, 256>(v, in, a, g, st, dtb, false, tid);                \
         stage_run<r, SIGN, R, 256>(v, st, a.tb, tid);                           \
-        stage_store<r, SIGN, R, 256, POST>(v, out, a, g, st, dtb, false, tid);  \
+        stage_store<r, SIGN, R, 256, false>(v, out, a, g, st, dtb, false, tid); \
     }
     MIXED_SWITCH(st.r, MIXED_ONE)
 }
