@@ -126,6 +126,12 @@ void mixed_schedule(MixedArgs &a, int prec)
     const int want = col ? 64 / eb : 1;
     a.tbp = 1;
     double best = 0;
+    // The smallest column passes are one block: what the passes beside it wrote and
+    // will read then stays in one L2.  complex64, in the blocks of least cost /
+    // in one (forward and inverse, rows and columns): 64 x 20 15.9 / 14.3 us,
+    // 16 x 24 14.3 / 12.6, FP64 64 x 18 16.1 / 15.3; even at 64 x 30 (16.8 /
+    // 16.1, FP64 17.1 / 17.5), no gain from 64 x 36 on.
+    const bool small = col && a.lines * a.n <= 2048;
     // the line count of least cost for threads of e elements
     auto tile = [&](int e, int cap, int nt, int most) {
         while (nt < (col ? 1024 : 512) && nt * cap < want * a.n) nt *= 2;
@@ -145,6 +151,7 @@ void mixed_schedule(MixedArgs &a, int prec)
             const double mem = seg < 24 ? 1.9 : seg < 32 ? 1.45 : seg < 64 ? 1.2 : 1.0;
             const double cost = (double)((blocks + slots - 1) / slots) * ((double)tb * a.n + 1000.0) * mem;
             if (best == 0 || cost < best) best = cost, a.tb = tb, a.tbp = tbp, a.nt = nt, a.e = e, a.cap = cap;
+            if (small && tb >= a.lines) break;
         }
     };
     if (a.nst == 1) {
