@@ -756,8 +756,8 @@ class Planner {
     // (kernels_chirp.hip).  M <= CHIRP_MAX_M: one in-place pass, each line's
     // convolution inside a workgroup (bluestein_lines).  Contiguous lines up
     // to M = CHIRP_ROWS_M: three passes through padded rows in the other
-    // buffer.  Else: chirp pre-multiply of every line into its own zero-padded row of M elements in the other buffer, forward FFT_M over
-    // the rows, product with the transformed filter of the direction,
+    // buffer.  Else: chirp pre-multiply of every line into its own zero-padded
+    // row of M elements in the other buffer, forward FFT_M over the rows, product with the transformed filter of the direction,
     // inverse FFT_M (both inner FFTs keep their direction whatever the outer
     // one), chirp post-multiply back into the line.  The data stays in
     // buffer *cur.  The filters are transformed here, at plan time, by a
@@ -1616,10 +1616,14 @@ int build_plan(struct topeFFT *f, int shape, long long nx, long long ny, long lo
         for (size_t i = 0; i < P->passes.size() && P->alt_pass < 0; ++i)
             if (P->passes[i].kind == PASS_AXIS && P->passes[i].in_buf == P->passes[i].out_buf) P->alt_pass = (int)i;
         // Out of place, the four-step's narrow tiles write 64-byte segments
-        // of two arrays: once those outgrow the cache, three passes of
+        // of two arrays: once one transform fills the cache, three passes of
         // short transforms in wide tiles take less time (1D FP64, forward +
         // inverse: 2^24 645 us against 700; 2^23 311 against 315, 2^22 165
-        // against 146)
+        // against 146).  Of the lengths of two passes that is FP64 2^24 alone:
+        // complex64 would need 2^25 points, which run three passes anyway.
+        // The line is drawn by the transform and not by a batch's array, as
+        // batches of shorter rows have not been measured both ways; nor
+        // has the plan's own array, which may end in its second buffer.
         if ((shape == 1 || shape == SHAPE_BATCH) && mode == MP_VALU && is_pow2(nx) && nx <= kMaxAxis &&
             nx * (long long)P->elem >= kCacheBytes) {
             std::vector<Pass> own;

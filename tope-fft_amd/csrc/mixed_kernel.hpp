@@ -16,16 +16,16 @@
 // radix are correctly rounded literals, so no device sin/cos is evaluated.
 //
 // What bounds it: the latency of a stage -- one exchange, its barriers and
-// its twiddles -- so the radices are as few as possible (mixed_plan), the
+// its twiddles -- so the radices are as few as possible (mixed_schedule), the
 // composite ones (6, 10, 12, 14, 15) are prime-factor DFTs without inner
 // twiddles, and a thread keeps its butterflies in registers over the
 // exchange, which leaves one LDS buffer instead of two and so twice the
 // blocks on a CU.
 // A forward and an inverse transform, against radices 2, 3, 4, 5, 7, 8, 16
 // between two LDS buffers with roots from a two-level table: 3000^2 648 ->
-// 323 us (rows 160 -> 74 us, 3.9 TB/s; columns 172 -> 92 us: a tile of three
+// 321 us (rows 160 -> 68 us, 4.2 TB/s; columns 172 -> 99 us: a tile of three
 // lines fills the LDS, so one block per CU alternates between memory and
-// arithmetic), 100^3 85 -> 63.5 us, 1000^2 52 us, complex64 100^3 45 us.
+// arithmetic), 100^3 85 -> 63.5 us, 1000^2 51 us, complex64 100^3 45 us.
 // Twiddles read ahead of the barrier before their stage: 1-3 % of that.
 #pragma once
 #include "internal.hpp"
@@ -41,7 +41,6 @@ struct Div32 {
     int d;
     float r;
 };
-__device__ __forceinline__ Div32 mkdiv(int d) { return Div32{d, 1.0f / (float)d}; }
 __device__ __forceinline__ int divmod(int a, const Div32 &d, int &rem)
 {
     int q = (int)((float)a * d.r);
@@ -235,7 +234,7 @@ __device__ __forceinline__ void stage_at(int bi, const Stage &st, const Div32 &d
 // the next.
 // Both are linear in i, so the r slots of a butterfly are one base and a
 // uniform stride.  Reads are contiguous over the lanes and so are the writes
-// but a first stage's, r slots apart: mixed_plan puts a radix first that
+// but a first stage's, r slots apart: mixed_schedule puts a radix first that
 // has few factors of two.
 template <bool COL>
 __device__ __forceinline__ int slot_of(int t, int i, int n, int tbp)
